@@ -547,7 +547,7 @@ __device__ __forceinline__ void solve_stream(int n, int m, const T* __restrict__
 #pragma unroll
     for (int s = 0; s < KS; ++s)
 #pragma unroll
-      for (int c = 0; c < MCT; ++c) acc[c] = fma_t(v[s], x[s * MCT + c], acc[c]);
+      for (int c = 0; c < MCT; ++c) acc[c] = __builtin_elementwise_fma(v[s], x[s * MCT + c], acc[c]);
 #pragma unroll
     for (int c = 0; c < MCT; ++c) {
       acc[c] += __shfl_xor(acc[c], 16);
