@@ -32,24 +32,40 @@ namespace {
 // right half's columns with it (one GEMM, rank = the left half's width, lower
 // part of the top square), factor the right half.  A kNB-wide block is the
 // diagonal block in LDS (with its inverse), then the rows below it as one MFMA
-// product with that inverse.  Against a kNB-at-a-time right-looking sweep the
+// product with that inverse.  (A panel of few rows goes by step launches instead;
+// *stepped tells whether its last block's L still waits beside its place.)  Against
+// a kNB-at-a-time right-looking sweep the
 // launches are as many, but each column of the panel is read and written by
 // log2(kb / kNB) updates instead of up to kb / kNB - 1, and the updates have rank
 // 64 .. 256 instead of 64.
 template <typename T>
 hipError_t factor_panel(T* a, int64_t lda, int n, int k0, int kb, int32_t* info, T* dinv, hipStream_t st,
-                        Profiler* prof, bool diag_f64) {
+                        Profiler* prof, bool diag_f64, bool* stepped) {
   const double es = (double)sizeof(T);
+  if (n - k0 <= step_rows<T>()) {
+    for (int k = k0; k < k0 + kb; k += kNB) {
+      const double db = std::min(kNB, n - k), below = std::max(0, n - k - kNB), pb = k > k0 ? db : 0.0;
+      const double cols = std::max(0, k0 + kb - k - kNB);
+      const double outs = below * cols - cols * (cols - 1.0) / 2.0;
+      LLH_PROF_ON(st, kDiagFactor, 2.0 * db * db * db / 3.0 + 2.0 * below * db * (db + pb) + 2.0 * outs * pb,
+                  es * (2.0 * db * db + below * (2.0 * db + pb) + (pb > 0.0 ? 2.0 * outs : 0.0)),
+                  (diag_f64 && sizeof(T) == 4
+                       ? launch_panel_step<T, double>(a, lda, n, k, k0, k0 + kb, dinv, info, *stepped, st)
+                       : launch_panel_step<T>(a, lda, n, k, k0, k0 + kb, dinv, info, *stepped, st)));
+      *stepped = true;
+    }
+    return hipSuccess;
+  }
   if (kb > kNB) {
     const int h = (kb / kNB + 1) / 2 * kNB;  // left half: a whole number of blocks, at least one
-    LLH_TRY(factor_panel<T>(a, lda, n, k0, h, info, dinv, st, prof, diag_f64));
+    LLH_TRY(factor_panel<T>(a, lda, n, k0, h, info, dinv, st, prof, diag_f64, stepped));
     const int below = n - k0 - h, cols = kb - h;  // rows k0+h.., columns k0+h .. k0+kb
     T* left = a + (int64_t)(k0 + h) * lda + k0;    // L of rows k0+h.., columns k0 .. k0+h
     const double outs = (double)below * cols - (double)cols * (cols - 1) / 2.0, dh = h;
     LLH_PROF_ON(st, kPanelUpdate, 2.0 * outs * dh, es * (2.0 * outs + ((double)below + cols) * dh),
                 (launch_gemm<T>(false, true, true, below, cols, h, T(-1), left, lda, left, lda, T(1), left + h, lda,
                                 info, st)));
-    return factor_panel<T>(a, lda, n, k0 + h, cols, info, dinv, st, prof, diag_f64);
+    return factor_panel<T>(a, lda, n, k0 + h, cols, info, dinv, st, prof, diag_f64, stepped);
   }
   const int k = k0, b = kb;
   T* akk = a + (int64_t)k * lda + k;
@@ -91,7 +107,7 @@ hipError_t trailing_syrk(int m, int kb, const T* p, int64_t lda, T* c, int32_t* 
 }  // namespace
 
 // Right-looking blocked Cholesky of the lower triangle (the blocked equivalent
-// of cholesky.rs:54-74).  Each outer panel (outer_width(n) columns) is factored
+// of cholesky.rs:54-74).  Each outer panel (panel_width() columns) is factored
 // by factor_panel; then one SYRK of that rank on MFMA updates the trailing matrix.
 // With lookahead, the trailing update of panel k is split: the next panel's
 // columns are updated and that panel factored on the side stream while the SYRK
@@ -131,21 +147,20 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
     LLH_TRY(launch_potrf_exact_single<T>(a, lda, n, info, 0, nullptr, s));
     if (dinv != nullptr) LLH_TRY(launch_trtri_blocks<T>(n, a, lda, false, false, dinv, info, s));
   } else {
-    const int nbo = outer_width(n, half != nullptr);
-    LLH_TRY(factor_panel<T>(a, lda, n, 0, std::min(nbo, n), info, dinv, s, prof, diag_f64));
+    const int kb0 = std::min(panel_width(n, n, half != nullptr), n);
+    bool stepped = false;  // the last block column was a step launch (its L_kk is still beside its place)
+    LLH_TRY(factor_panel<T>(a, lda, n, 0, kb0, info, dinv, s, prof, diag_f64, &stepped));
     if (ff != nullptr) {
       LLH_TRY(hipEventRecord(la->fwd_ev, s));
       LLH_TRY(hipStreamWaitEvent(la->fwd, la->fwd_ev, 0));
       if (ff->b != nullptr)
         LLH_TRY(hipMemcpy2DAsync(ff->y, ff->ldy * sizeof(T), ff->b, ff->ldb * sizeof(T), ff->m * sizeof(T), n,
                                  hipMemcpyDeviceToDevice, la->fwd));
-      LLH_TRY(fwd_panel(0, std::min(nbo, n)));
+      LLH_TRY(fwd_panel(0, kb0));
     }
-    for (int k0 = 0; k0 < n; k0 += nbo) {
-      const int kb = std::min(nbo, n - k0);
+    for (int k0 = 0, kb = kb0, kb2 = 0; k0 + kb < n; k0 += kb, kb = kb2) {
       const int m2 = n - k0 - kb;
-      if (m2 <= 0) break;
-      const int kb2 = std::min(nbo, m2);  // width of the next panel
+      kb2 = std::min(panel_width(m2, n, half != nullptr), m2);  // width of the next panel
       T* p = a + (int64_t)(k0 + kb) * lda + k0;  // L21: rows k0+kb.., columns k0..k0+kb
       T* c = p + kb;                              // trailing matrix at (k0+kb, k0+kb)
       // The trailing SYRK's algorithmic work: outs outputs of the lower
@@ -155,7 +170,7 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
         const double outs = (double)m2 * (m2 + 1) / 2.0;
         LLH_PROF(kTrailingSyrk, 2.0 * outs * kb, es * 2.0 * outs + pes * (double)m2 * kb,
                  (trailing_syrk<T>(m2, kb, p, lda, c, info, half, s)));
-        LLH_TRY(factor_panel<T>(a, lda, n, k0 + kb, kb2, info, dinv, s, prof, diag_f64));
+        LLH_TRY(factor_panel<T>(a, lda, n, k0 + kb, kb2, info, dinv, s, prof, diag_f64, &stepped));
         continue;
       }
       // With half, the whole panel (m2 x kb) is rounded to f16 once, before the
@@ -183,7 +198,7 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
                       (launch_gemm<T>(false, true, true, m2, kb2, kb, T(-1), p, lda, p, lda, T(1), c, lda, info,
                                       la->side)));
         }
-        LLH_TRY(factor_panel<T>(a, lda, n, k0 + kb, kb2, info, dinv, la->side, prof, diag_f64));
+        LLH_TRY(factor_panel<T>(a, lda, n, k0 + kb, kb2, info, dinv, la->side, prof, diag_f64, &stepped));
       }
       LLH_TRY(hipEventRecord(la->join, la->side));
       if (ff != nullptr) {
@@ -298,7 +313,7 @@ hipError_t solve_pair_enqueue(int n, const T* a, int64_t lda, int m, T* b, int64
 
 template <typename T>
 bool forward_fusable(int n, int m, const Lookahead* la) {
-  return m > 0 && m <= 64 && n > outer_width(n, false) && n > kSolvePairLdsMaxN && n > small_max<T>() &&
+  return m > 0 && m <= 64 && n > panel_width(n, n, false) && n > kSolvePairLdsMaxN && n > small_max<T>() &&
          la != nullptr && la->fwd != nullptr && la->fwd_ev != nullptr;
 }
 

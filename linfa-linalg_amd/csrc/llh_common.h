@@ -32,6 +32,23 @@ constexpr int kNBO_LARGE = 1024;
 constexpr int kNBO_LARGE_N = 24576;
 inline int outer_width(int n, bool half_syrk) { return (!half_syrk && n >= kNBO_LARGE_N) ? kNBO_LARGE : kNBO; }
 
+// The last kStepTail columns are one panel (their updates ride on the step
+// launches below), those before it outer_width panels.  Measured (potrf, us) with a tail of 2048 / 4096 / 6144:
+// f64 n = 3000 1106 / 952, 5003 2561 / 2580 / 2601, 8192 5894 / 5952 / 6930; f32
+// n = 3000 835 / 756, 5003 1960 / 1890 / 1886, 8192 3882 / 3898 / 4455.
+constexpr int kStepTail = 4096;
+inline int panel_width(int rem, int n, bool half_syrk) { return rem <= kStepTail ? rem : outer_width(n, half_syrk); }
+
+// A panel whose rows number at most step_rows is factored by one launch per 64
+// columns (launch_panel_step), in which every workgroup repeats the diagonal
+// block; with more rows than that the repeated work and its rank-64 updates take
+// more from the trailing SYRK beside them than the shorter chain gives.  Measured (potrf, ms)
+// with bounds of 0 / 4096 / 8192 / 16384 rows (512-wide panels): f64 n = 8192 7.2 / 6.6 /
+// 6.2, 16384 32.7 / 32.0 / 31.5 / 31.9; f32 n = 12000 10.3 / 9.7 / 9.1 / 8.8, 16384
+// 19.7 / 19.0 / 18.5 / 18.3.
+template <typename T>
+constexpr int step_rows() { return sizeof(T) == 8 ? 8192 : 16384; }
+
 // Right-hand-side columns per workgroup of the one-launch triangular solve, and
 // the bound on its flag waits (2^22 polls: well over 0.1 s, far above any real wait).
 constexpr int kSolveChunkHost = 16;

@@ -148,6 +148,15 @@ int med_resident_per_cu(bool solve);
 template <typename TS, typename T = TS>
 hipError_t launch_diag_fast(TS* a, int64_t lda, int b, TS* inv, int32_t* info, int64_t info_base,
                             const int32_t* gate, hipStream_t s);
+// k_step.hip: block column k0 of the panel [p0, kend) in one launch: column k0 - 64
+// applied to columns [k0, kend) (k0 > p0), the diagonal block factored and
+// inverted (dinv: the inverses of all blocks), and the rows below multiplied by
+// that inverse.  L of the diagonal block waits in the next block's slot of dinv
+// for the next launch, which puts it in its place when copy_prev is set (set it
+// on every launch but the first of a sequence).
+template <typename TS, typename T = TS>
+hipError_t launch_panel_step(TS* a, int64_t lda, int n, int k0, int p0, int kend, TS* dinv, int32_t* info,
+                             bool copy_prev, hipStream_t s);
 // k_diag.hip: grouped form over step work (factor + inverse of each block).
 template <typename T>
 hipError_t launch_grp_diag_fast(const BatchBase<T>* base, const BatchItem* items, const StepWork* work,
