@@ -76,27 +76,45 @@ __global__ __launch_bounds__(256) void gram_partial_kernel(int n, int ka, int kb
         P[(la + 16 * i + MF::row(lane, e)) * kGramTile + lb + 16 * j + m] = acc[i][j][e];
 }
 
-// C[a][b] = sum over chunks, in chunk order, of the partial tiles.
+// C[a][b] = the sum over chunks of the partial tiles: 64 outputs per workgroup
+// (one per lane), the chunks dealt to its 16 waves, whose sums are added in wave
+// order -- a fixed order, whatever the scheduling.  With one thread per output
+// walking all chunks, 2048 dependent loads took 663 us for a 64 x 64 product
+// (chunks of 512 rows); this way 25.
+constexpr int kGramWaves = 16;
 template <typename T>
-__global__ void gram_reduce_kernel(int chunks, int tiles_a, int tiles_b, int ka, int kb,
-                                   const T* __restrict__ partial, T* __restrict__ C, int64_t ldc) {
-  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (e >= (int64_t)ka * kb) return;
-  const int a = (int)(e / kb), b = (int)(e % kb);
+__global__ __launch_bounds__(64 * kGramWaves) void gram_reduce_kernel(int chunks, int tiles_a, int tiles_b, int ka,
+                                                                      int kb, const T* __restrict__ partial,
+                                                                      T* __restrict__ C, int64_t ldc) {
+  __shared__ T sum[kGramWaves][64];
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t e = (int64_t)blockIdx.x * 64 + lane;
+  const int64_t ec = min(e, (int64_t)ka * kb - 1);
+  const int a = (int)(ec / kb), b = (int)(ec % kb);
   const int ta = a / kGramTile, tb = b / kGramTile, off = (a % kGramTile) * kGramTile + b % kGramTile;
   const int64_t stride = (int64_t)tiles_a * tiles_b * kGramTile * kGramTile;
   const T* p = partial + ((int64_t)ta * tiles_b + tb) * kGramTile * kGramTile + off;
   T s = T(0);
-  for (int c = 0; c < chunks; ++c) s += p[c * stride];
-  C[(int64_t)a * ldc + b] = s;
+#pragma unroll 8
+  for (int c = wave; c < chunks; c += kGramWaves) s += p[c * stride];
+  sum[wave][lane] = s;
+  __syncthreads();
+  if (wave == 0 && e < (int64_t)ka * kb) {
+    T t = sum[0][lane];
+#pragma unroll
+    for (int w = 1; w < kGramWaves; ++w) t += sum[w][lane];
+    C[(int64_t)a * ldc + b] = t;
+  }
 }
 
 }  // namespace
 
 int64_t gram_partial_elems(int n, int ka, int kb, int* chunks, int* rows_per_chunk) {
   const int tiles_a = (ka + kGramTile - 1) / kGramTile, tiles_b = (kb + kGramTile - 1) / kGramTile;
-  // about 2048 workgroups, at least 256 rows (16 MFMA iterations) each
-  const int want = std::max(1, 2048 / (tiles_a * tiles_b));
+  // about 1024 workgroups (16 waves a CU; 2048 write and read twice the partial
+  // tiles: 1646 against 1623 us for apply_constraints and orthonormalize of a
+  // 2^20 x 64 block), at least 256 rows (16 MFMA iterations) each
+  const int want = std::max(1, 1024 / (tiles_a * tiles_b));
   int rpc = (n + want - 1) / want;
   rpc = std::max(256, (rpc + 15) / 16 * 16);
   *rows_per_chunk = rpc;
@@ -119,7 +137,7 @@ hipError_t launch_gram(int n, int ka, int kb, const T* A, int64_t lda, const T* 
   hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
   const int64_t total = (int64_t)ka * kb;
-  hipLaunchKernelGGL((gram_reduce_kernel<T>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, chunks, tiles_a,
+  hipLaunchKernelGGL((gram_reduce_kernel<T>), dim3((unsigned)((total + 63) / 64)), dim3(64 * kGramWaves), 0, s, chunks, tiles_a,
                      tiles_b, ka, kb, partial, C, ldc);
   return hipGetLastError();
 }

@@ -34,6 +34,19 @@ __global__ void is_triangular_kernel(const T* a, int64_t lda, int n, bool upper,
   if (other && !(a[(int64_t)r * lda + c] == T(0))) *flag = 0;
 }
 
+// dst[c][r] = src[r][c], 32 x 32 tiles through LDS.
+template <typename T>
+__global__ __launch_bounds__(256) void transpose_kernel(int rows, int cols, const T* __restrict__ src, int64_t lds,
+                                                        T* __restrict__ dst, int64_t ldd) {
+  __shared__ T tile[32][33];
+  const int r0 = blockIdx.y * 32, c0 = blockIdx.x * 32, tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
+  for (int y = ty; y < 32; y += 8)
+    if (r0 + y < rows && c0 + tx < cols) tile[y][tx] = src[(int64_t)(r0 + y) * lds + c0 + tx];
+  __syncthreads();
+  for (int y = ty; y < 32; y += 8)
+    if (c0 + y < cols && r0 + tx < rows) dst[(int64_t)(c0 + y) * ldd + r0 + tx] = tile[tx][y];
+}
+
 // a[r][c] = a[c][r] for c > r: the upper triangle mirrors the lower.  One
 // 32 x 32 tile pair per workgroup (tile (ti, tj), tj >= ti, receives the
 // transpose of tile (tj, ti)), staged through LDS so reads and writes are both
@@ -122,6 +135,14 @@ hipError_t launch_set_identity(T* a, int64_t lda, int n, hipStream_t s) {
 }
 
 template <typename T>
+hipError_t launch_transpose(int rows, int cols, const T* src, int64_t lds, T* dst, int64_t ldd, hipStream_t s) {
+  if (rows <= 0 || cols <= 0) return hipSuccess;
+  hipLaunchKernelGGL((transpose_kernel<T>), dim3((cols + 31) / 32, (rows + 31) / 32), dim3(256), 0, s, rows, cols, src,
+                     lds, dst, ldd);
+  return hipGetLastError();
+}
+
+template <typename T>
 hipError_t launch_mirror_lower(T* a, int64_t lda, int n, hipStream_t s) {
   if (n <= 1) return hipSuccess;
   const int64_t nt = (n + 31) / 32;
@@ -150,6 +171,8 @@ template hipError_t launch_copy_rows_gated<double>(int, int, const double*, int6
                                                    const int32_t*, hipStream_t);
 template hipError_t launch_copy_rows_gated<float>(int, int, const float*, int64_t, float*, int64_t, const int32_t*,
                                                   hipStream_t);
+template hipError_t launch_transpose<double>(int, int, const double*, int64_t, double*, int64_t, hipStream_t);
+template hipError_t launch_transpose<float>(int, int, const float*, int64_t, float*, int64_t, hipStream_t);
 template hipError_t launch_mirror_lower<double>(double*, int64_t, int, hipStream_t);
 template hipError_t launch_mirror_lower<float>(float*, int64_t, int, hipStream_t);
 template hipError_t launch_copy_lower<double>(int, const double*, int64_t, double*, int64_t, hipStream_t);
