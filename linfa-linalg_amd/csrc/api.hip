@@ -149,6 +149,7 @@ hipError_t ctx_sync(llh_context* ctx, int n, int m, SolveSync* sync) {
   sync->nflags = (int64_t)(ctx->sync.bytes / sizeof(int32_t)) - 2;
   sync->epoch = &ctx->epoch;
   sync->spin_limit = ctx->spin_limit;
+  sync->wild = ctx->d_info + 1;
   // one error word per call: cleared here, read back once the call's sweeps are done
   return solve_sync_begin(*sync, ctx->stream);
 }
@@ -165,6 +166,16 @@ hipError_t ctx_read_solve_error(llh_context* ctx) {
 }  // namespace llh
 
 namespace {
+
+// Whether a triangular solve of m columns left B untouched because a diagonal
+// block's inverse is not to be used (trsm_enqueue); the context's stream has been
+// waited for, ctx->h_info[1] read with ctx_read_solve_wild.
+bool solve_wild(const llh_context* ctx, size_t m) { return m > 64 && ctx->h_info[1] != kNoFail; }
+hipError_t ctx_read_solve_wild(llh_context* ctx, size_t m) {
+  ctx->h_info[1] = kNoFail;
+  if (m <= 64 || m > (size_t)kSolveMaxCols) return hipSuccess;
+  return hipMemcpyAsync(ctx->h_info + 1, ctx->d_info + 1, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream);
+}
 
 llh_status solve_stalled(llh_error* err) {
   return set_error(err, LLH_ERR_HIP, 0, 0, -1, "triangular solve: a block wait exceeded its bound", 0);
@@ -396,10 +407,18 @@ llh_status solve_triangular_plain(llh_context* ctx, size_t rows, size_t cols, co
                             ctx->profiler()),
             "trsm");
   CHECK_HIP(ctx_read_solve_error(ctx), "solve status");
+  CHECK_HIP(ctx_read_solve_wild(ctx, b_cols), "solve status");
   CHECK_HIP(hipMemcpyAsync(hb, db, n * b_cols * sizeof(T), hipMemcpyDeviceToHost, ctx->stream),
             "download");
   CHECK_HIP(hipStreamSynchronize(ctx->stream), "synchronize");
   if (ctx->h_info[2] != 0) return solve_stalled(err);
+  if (solve_wild(ctx, b_cols)) {
+    CHECK_HIP(trsm_enqueue<T>(uplo == LLH_UPPER, false, (int)n, da, (int64_t)n, (int)b_cols, db, (int64_t)b_cols,
+                              nullptr, false, nullptr, nullptr, ctx->stream, ctx->profiler()),
+              "trsm");
+    CHECK_HIP(hipMemcpyAsync(hb, db, n * b_cols * sizeof(T), hipMemcpyDeviceToHost, ctx->stream), "download");
+    CHECK_HIP(hipStreamSynchronize(ctx->stream), "synchronize");
+  }
   scatter(hb, n, b_cols, b, brs, bcs, [b_cols](size_t) { return b_cols; });
   return ok(err);
 }
@@ -577,8 +596,15 @@ llh_status dev_solve_triangular(llh_context* ctx, llh_uplo uplo, int trans, size
                             nullptr, false, static_cast<T*>(dinv), &sync, ctx->stream, ctx->profiler()),
             "trsm");
   CHECK_HIP(ctx_read_solve_error(ctx), "solve status");
+  CHECK_HIP(ctx_read_solve_wild(ctx, m), "solve status");
   CHECK_HIP(hipStreamSynchronize(ctx->stream), "synchronize");
   if (ctx->h_info[2] != 0) return solve_stalled(err);
+  if (solve_wild(ctx, m)) {
+    CHECK_HIP(trsm_enqueue<T>(uplo == LLH_UPPER, trans != 0, (int)n, a, (int64_t)lda, (int)m, b, (int64_t)ldb,
+                              nullptr, false, nullptr, nullptr, ctx->stream, ctx->profiler()),
+              "trsm");
+    CHECK_HIP(hipStreamSynchronize(ctx->stream), "synchronize");
+  }
   return ok(err);
 }
 
@@ -721,18 +747,22 @@ llh_status dev_apply_constraints(llh_context* ctx, size_t n, size_t k, T* v, siz
     return invalid(err, "bad matrix arguments");
   if (n > 0x7fffffff || k > 0x7fffffff || ky > 0x7fffffff) return invalid(err, "matrix too large");
   const int N = (int)n, K = (int)k, KY = (int)ky;
-  T *part = nullptr, *g = nullptr, *unused = nullptr;
-  CHECK_HIP(lobpcg_scratch<T>(ctx, N, KY, K, 0, &part, &g, &unused), "scratch");
+  T *part = nullptr, *g = nullptr, *gt = nullptr;
+  CHECK_HIP(lobpcg_scratch<T>(ctx, N, KY, K, ky * k, &part, &g, &gt), "scratch");
   hipStream_t s = ctx->stream;
   CHECK_HIP(launch_gram<T>(N, KY, K, y, (int64_t)ldy, v, (int64_t)ldv, g, (int64_t)K, part, s), "gram");
   void* dv = nullptr;
   CHECK_HIP(ctx_dinv(ctx, KY, sizeof(T), &dv), "inverse buffer");
   SolveSync sync;
   CHECK_HIP(ctx_sync(ctx, KY, K, &sync), "solve sync");
+  sync.wild = nullptr;  // (its answer is not waited for here: k > 64 solves by substitution)
   CHECK_HIP(trsm_enqueue<T>(false, false, KY, l_yy, (int64_t)ldl, K, g, (int64_t)K, nullptr, false,
                             static_cast<T*>(dv), &sync, s, ctx->profiler()),
             "solve");
-  CHECK_HIP(launch_gemm<T>(false, false, false, N, K, KY, T(-1), y, (int64_t)ldy, g, (int64_t)K, T(1), v,
+  // u transposed, so that the tall product's operands are both contiguous along
+  // the sum (2^20 x 64 in f64: 510 us with u as it is, 320 so)
+  CHECK_HIP(launch_transpose<T>(KY, K, g, (int64_t)K, gt, (int64_t)KY, s), "transpose");
+  CHECK_HIP(launch_gemm<T>(false, true, false, N, K, KY, T(-1), y, (int64_t)ldy, gt, (int64_t)KY, T(1), v,
                            (int64_t)ldv, nullptr, s),
             "update");
   CHECK_HIP(ctx_read_solve_error(ctx), "solve status");

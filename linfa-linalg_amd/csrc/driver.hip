@@ -230,6 +230,46 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
   return hipSuccess;
 }
 
+namespace {
+
+// op(A) X = B with the inverses of the diagonal blocks: one launch
+// (launch_trsm_persistent) up to solve_split<T>(m) rows, otherwise by halves: the
+// half that comes first, one product into the other half's rows, the other half.
+template <typename T>
+hipError_t trsm_split(bool upper_op, bool trans, int n, const T* a, int64_t lda, int m, T* b, int64_t ldb,
+                      const T* dinv, bool dinv_t, SolveSync* sync, hipStream_t s, Profiler* prof,
+                      const int32_t* gate) {
+  const double es = (double)sizeof(T);
+  if (n <= solve_split<T>(m)) {
+    // the launcher resets the ticket; the error word is the call's (solve_sync_begin)
+    const int32_t epoch = (*sync->epoch)++;
+    const double fl = (double)n * n * m;
+    LLH_PROF(kSolveGemm, fl, es * ((double)n * n / 2.0 + 2.0 * n * m),
+             (launch_trsm_persistent<T>(n, m, a, lda, trans, !upper_op, dinv, dinv_t, b, ldb, sync->words,
+                                        sync->words + 2, epoch, sync->words + 1, sync->spin_limit, gate, s)));
+    return hipSuccess;
+  }
+  const int n1 = ((n + kNB - 1) / kNB + 1) / 2 * kNB, n2 = n - n1;
+  const T* d2 = dinv + (int64_t)(n1 / kNB) * kNB * kNB;
+  const T* a22 = a + (int64_t)n1 * lda + n1;
+  T* b2 = b + (int64_t)n1 * ldb;
+  const double fl = 2.0 * n1 * n2 * m, by = es * ((double)n1 * n2 + 2.0 * n * m);
+  if (!upper_op) {
+    LLH_TRY(trsm_split<T>(upper_op, trans, n1, a, lda, m, b, ldb, dinv, dinv_t, sync, s, prof, gate));
+    LLH_PROF(kSolveGemm, fl, by,
+             (launch_gemm<T>(trans, false, false, n2, m, n1, T(-1), trans ? a + n1 : a + (int64_t)n1 * lda, lda, b,
+                             ldb, T(1), b2, ldb, gate, s)));
+    return trsm_split<T>(upper_op, trans, n2, a22, lda, m, b2, ldb, d2, dinv_t, sync, s, prof, gate);
+  }
+  LLH_TRY(trsm_split<T>(upper_op, trans, n2, a22, lda, m, b2, ldb, d2, dinv_t, sync, s, prof, gate));
+  LLH_PROF(kSolveGemm, fl, by,
+           (launch_gemm<T>(trans, false, false, n1, m, n2, T(-1), trans ? a + (int64_t)n1 * lda : a + n1, lda, b2,
+                           ldb, T(1), b, ldb, gate, s)));
+  return trsm_split<T>(upper_op, trans, n1, a, lda, m, b, ldb, dinv, dinv_t, sync, s, prof, gate);
+}
+
+}  // namespace
+
 // Blocked substitution for op(A) X = B (B row-major n x m, in place), kNB rows
 // at a time: solve the diagonal block, then subtract its contribution from the
 // rows still to come with one GEMM (the column sweep of triangular.rs:113-125,
@@ -240,23 +280,24 @@ hipError_t trsm_enqueue(bool upper_op, bool trans, int n, const T* a, int64_t ld
                         Profiler* prof, const int32_t* gate) {
   if (n <= 0 || m <= 0) return hipSuccess;
   const double es = (double)sizeof(T);
-  const int nblk0 = (n + kNB - 1) / kNB;
-  const int nq = (m + kSolveChunkHost - 1) / kSolveChunkHost;
-  if (sync != nullptr && sync->epoch != nullptr && m <= 64 && sync->nflags >= (int64_t)nblk0 * nq &&
-      (dinv != nullptr || dinv_work)) {
+  if (sync != nullptr && sync->epoch != nullptr && m <= kSolveMaxCols && sync->nflags >= solve_flags<T>(n, m) &&
+      (dinv != nullptr || (dinv_work != nullptr && (m <= 64 || sync->wild != nullptr)))) {
     if (dinv == nullptr) {
+      // Above 64 columns the caller looks at *wild afterwards and, where a
+      // diagonal block is singular or its inverse large, takes the substitution
+      // below instead (this path then leaves B untouched).
+      int32_t* wild = m > 64 ? sync->wild : nullptr;
+      if (wild != nullptr) {
+        if (gate != nullptr) return hipErrorInvalidValue;
+        LLH_TRY(launch_fill_i32(wild, kNoFail, 1, s));
+        gate = wild;
+      }
       LLH_PROF(kSolveDiag, (double)n * kNB * kNB / 3.0, es * (double)n * kNB,
-               (launch_trtri_blocks<T>(n, a, lda, trans, upper_op, dinv_work, gate, s)));
+               (launch_trtri_blocks<T>(n, a, lda, trans, upper_op, dinv_work, nullptr, s, wild)));
       dinv = dinv_work;
       dinv_t = false;
     }
-    // the launcher resets the ticket; the error word is the call's (solve_sync_begin)
-    const int32_t epoch = (*sync->epoch)++;
-    const double fl = (double)n * n * m;
-    LLH_PROF(kSolveGemm, fl, es * ((double)n * n / 2.0 + 2.0 * n * m),
-             (launch_trsm_persistent<T>(n, m, a, lda, trans, !upper_op, dinv, dinv_t, b, ldb, sync->words,
-                                        sync->words + 2, epoch, sync->words + 1, sync->spin_limit, gate, s)));
-    return hipSuccess;
+    return trsm_split<T>(upper_op, trans, n, a, lda, m, b, ldb, dinv, dinv_t, sync, s, prof, gate);
   }
   const int nblk = (n + kNB - 1) / kNB;
   if (!upper_op) {  // forward

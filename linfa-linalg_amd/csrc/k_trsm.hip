@@ -109,11 +109,15 @@ __global__ __launch_bounds__(64) void trsv_block_kernel(int b, bool trans, const
     if (r < b) Y[(int64_t)r * ldy + col] = y[r];
 }
 
-// trtri64: one workgroup per diagonal block (trtri64_block, k_trsm_impl.h).
+// trtri64: one workgroup per diagonal block (trtri64_block, k_trsm_impl.h).  A
+// block times its inverse is off by at most about 64 max |M| max |M^-1| eps, which a
+// substitution would not be: with `wild`, blocks beyond this bound are reported.
+// (Factors of SPD matrices with condition 4e6 stay below 4e3.)
+constexpr double kTameInverse = 4096.0;
 template <typename TS, typename T>
 __global__ __launch_bounds__(256) void trtri64_kernel(int n, const TS* __restrict__ A, int64_t lda, bool trans,
                                                       bool upper, TS* __restrict__ out,
-                                                      const int32_t* __restrict__ gate) {
+                                                      const int32_t* __restrict__ gate, int32_t* wild) {
   if (gate != nullptr && *gate != kNoFail) return;
   __shared__ T Ms[kNB * (kNB + 1)];
   __shared__ T Xs[kNB * (kNB + 1)];
@@ -121,6 +125,33 @@ __global__ __launch_bounds__(256) void trtri64_kernel(int n, const TS* __restric
   const int o = blockIdx.x * kNB;
   trtri64_block<TS, TS, T>(min(kNB, n - o), A + (int64_t)o * lda + o, lda, trans, upper,
                        out + (int64_t)blockIdx.x * kNB * kNB, Ms, Xs, Ts);
+  if (wild == nullptr) return;
+  // *wild := this block unless max |M| max |M^-1| <= kTameInverse (NaN and
+  // infinities fail it too)
+  __shared__ T red[2][4];
+  T mm = T(0), mx = T(0);
+  for (int e = threadIdx.x; e < kNB * kNB; e += 256) {
+    const int at = (e / kNB) * (kNB + 1) + e % kNB;
+    const T v = fabs(Ms[at]), x = fabs(Xs[at]);
+    mm = v > mm || v != v ? v : mm;  // (a NaN is taken, and kept)
+    mx = x > mx || x != x ? x : mx;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    const T v = __shfl_xor(mm, o), x = __shfl_xor(mx, o);
+    mm = v > mm || v != v ? v : mm;
+    mx = x > mx || x != x ? x : mx;
+  }
+  if ((threadIdx.x & 63) == 0) {
+    red[0][threadIdx.x >> 6] = mm;
+    red[1][threadIdx.x >> 6] = mx;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    bool tame = true;
+    for (int i = 0; i < 4; ++i)
+      for (int j = 0; j < 4; ++j) tame = tame && red[0][i] * red[1][j] <= T(kTameInverse);
+    if (!tame) atomicMin(wild, (int32_t)blockIdx.x);
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -437,10 +468,10 @@ hipError_t launch_trsv_block(bool upper_op, bool trans, int b, const T* Tm, int6
 
 template <typename TS, typename T>
 hipError_t launch_trtri_blocks(int n, const TS* A, int64_t lda, bool trans, bool upper, TS* out,
-                               const int32_t* gate, hipStream_t s) {
+                               const int32_t* gate, hipStream_t s, int32_t* wild) {
   if (n <= 0) return hipSuccess;
   hipLaunchKernelGGL((trtri64_kernel<TS, T>), dim3((n + kNB - 1) / kNB), dim3(256), 0, s, n, A, lda, trans,
-                     upper, out, gate);
+                     upper, out, gate, wild);
   return hipGetLastError();
 }
 
@@ -464,11 +495,11 @@ hipError_t launch_trsm_persistent(int n, int m, const T* A, int64_t lda, bool tr
 }
 
 template hipError_t launch_trtri_blocks<double, double>(int, const double*, int64_t, bool, bool, double*,
-                                                        const int32_t*, hipStream_t);
+                                                        const int32_t*, hipStream_t, int32_t*);
 template hipError_t launch_trtri_blocks<float, float>(int, const float*, int64_t, bool, bool, float*,
-                                                      const int32_t*, hipStream_t);
+                                                      const int32_t*, hipStream_t, int32_t*);
 template hipError_t launch_trtri_blocks<float, double>(int, const float*, int64_t, bool, bool, float*,
-                                                       const int32_t*, hipStream_t);
+                                                       const int32_t*, hipStream_t, int32_t*);
 template hipError_t launch_trsm_persistent<double>(int, int, const double*, int64_t, bool, bool, const double*,
                                                    bool, double*, int64_t, int32_t*, int32_t*, int32_t, int32_t*,
                                                    int64_t, const int32_t*, hipStream_t);

@@ -54,6 +54,28 @@ constexpr int step_rows() { return sizeof(T) == 8 ? 8192 : 16384; }
 constexpr int kSolveChunkHost = 16;
 constexpr int64_t kSpinLimit = 1ll << 22;
 
+// Rows that one launch of the triangular solve takes for m right-hand sides
+// (trsm_split): all of them up to 64 columns, where the chain of 64-row hops
+// bounds it; with more columns about as many as keep its products, which run on
+// the VALU, shorter than that chain -- n * m = 1.5M (f64), 3M (f32), the rest as
+// MFMA products between launches.  Measured (us) at 1024 / 2048 / 4096 rows / all:
+// f64 n = 4096 m = 300 1390 / 1063 / 873 / 869, m = 1500 2523 / 2749 / 3607 / 3606;
+// f64 n = 12000 m = 100 5304 / 4274 / 3416 / 2300, m = 500 6202 / 5162 / 4951 / 8342;
+// f32 n = 12000 m = 1500 8009 / 7292 / 7094 / 9491.
+constexpr int kSolveMaxCols = 32768;
+template <typename T>
+inline int solve_split(int m) {
+  if (m <= 64) return INT32_MAX;
+  const int rows = (sizeof(T) == 8 ? 1500000 : 3000000) / m / kNB * kNB;
+  return rows > kNB ? rows : kNB;
+}
+// Flags that the largest of those launches needs for order n.
+template <typename T>
+inline int64_t solve_flags(int n, int m) {
+  const int64_t nb = (n + kNB - 1) / kNB, per = (int64_t)solve_split<T>(m) / kNB;
+  return (nb < per ? nb : per) * ((m + kSolveChunkHost - 1) / kSolveChunkHost);
+}
+
 // Largest n the single-workgroup LDS kernel takes (the packed lower triangle of
 // an f64 matrix must fit in 160 KiB of LDS with room to spare).
 constexpr int kSmallMaxD = 128;

@@ -18,6 +18,9 @@ struct SolveSync {
   int64_t nflags = 0;
   int32_t* epoch = nullptr;
   int64_t spin_limit = kSpinLimit;  // bound on each flag wait (negative: give up at once)
+  // Device word of solves of more than 64 columns with inverses of their own
+  // (trsm_enqueue): kNoFail, or a diagonal block whose inverse is not to be used.
+  int32_t* wild = nullptr;
 };
 
 // Enqueues the clearing of the solve error word: once per call, before its

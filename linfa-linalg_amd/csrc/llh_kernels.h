@@ -218,7 +218,7 @@ hipError_t launch_trsv_block(bool upper_op, bool trans, int b, const T* Tm, int6
 // as consecutive row-major 64 x 64 blocks at out; upper names op(A)'s triangle.
 template <typename TS, typename T = TS>
 hipError_t launch_trtri_blocks(int n, const TS* A, int64_t lda, bool trans, bool upper, TS* out,
-                               const int32_t* gate, hipStream_t s);
+                               const int32_t* gate, hipStream_t s, int32_t* wild = nullptr);
 // k_trsm.hip: one-launch blocked solve op(A) X = B (B row-major n x m) using the
 // diagonal-block inverses Dinv (transposed when dinv_t).  ticket/flags/err are
 // device words (flags: one per 64-row block and 16-column chunk), epoch a value
@@ -268,6 +268,8 @@ hipError_t launch_is_triangular(const T* a, int64_t lda, int n, bool upper, int3
 template <typename T>
 hipError_t launch_set_identity(T* a, int64_t lda, int n, hipStream_t s);
 // a's strict upper triangle := the transpose of its strict lower triangle.
+template <typename T>
+hipError_t launch_transpose(int rows, int cols, const T* src, int64_t lds, T* dst, int64_t ldd, hipStream_t s);
 template <typename T>
 hipError_t launch_mirror_lower(T* a, int64_t lda, int n, hipStream_t s);
 // dst (m x m) := the lower triangle of src with zeros above it.
