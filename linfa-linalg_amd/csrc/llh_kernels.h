@@ -267,14 +267,17 @@ template <typename T>
 hipError_t launch_is_triangular(const T* a, int64_t lda, int n, bool upper, int32_t* flag, hipStream_t s);
 template <typename T>
 hipError_t launch_set_identity(T* a, int64_t lda, int n, hipStream_t s);
-// a's strict upper triangle := the transpose of its strict lower triangle.
+// dst (cols x rows) := the transpose of src (rows x cols).
 template <typename T>
 hipError_t launch_transpose(int rows, int cols, const T* src, int64_t lds, T* dst, int64_t ldd, hipStream_t s);
+// k_inv.hip: W = L^-1 (lower triangle of w) from its diagonal blocks, the level of
+// blocks of h rows (tmp: see potri_tmp_elems), and x := W^T W, both triangles.
 template <typename T>
-hipError_t launch_mirror_lower(T* a, int64_t lda, int n, hipStream_t s);
-// dst (m x m) := the lower triangle of src with zeros above it.
+hipError_t launch_inv_diag(int n, const T* dinv, T* w, int64_t ldw, hipStream_t s);
 template <typename T>
-hipError_t launch_copy_lower(int m, const T* src, int64_t lds, T* dst, int64_t ldd, hipStream_t s);
+hipError_t launch_inv_level(int n, int h, const T* l, int64_t lda, T* w, int64_t ldw, T* tmp, hipStream_t s);
+template <typename T>
+hipError_t launch_inv_wtw(int n, const T* w, int64_t ldw, T* x, int64_t ldx, hipStream_t s);
 // dst (rows x m, ldd) := src (lds), skipped whole once gate holds a failed row.
 template <typename T>
 hipError_t launch_copy_rows_gated(int rows, int m, const T* src, int64_t lds, T* dst, int64_t ldd,
