@@ -17,6 +17,8 @@
 //   A operand: lane l holds op(A)[l%16][k0 + l/16]
 //   B operand: lane l holds op(B)[k0 + l/16][l%16]
 //   f64 result reg i: C[4*i + l/16][l%16];  f32 result reg i: C[4*(l/16) + i][l%16]
+#include <algorithm>
+
 #include "llh_common.h"
 #include "llh_kernels.h"
 #include "k_gemm_impl.h"
@@ -242,22 +244,190 @@ __global__ __launch_bounds__(WM* WN * 64, (512 / (WM * WN * 64)) > 0 ? 512 / (WM
   const int m0 = tm * BM, n0 = tn * BN;
   if (TRI && m0 + BM - 1 < n0) return;
 
-  // C prefetch for the triangular updates (the trailing SYRK and the look-ahead
-  // panel's columns): f64 on 256 x 128 tiles (the 128 x 128 f64 tile has no
-  // registers left) and on 64 x 64 tiles (the small blocked factors' updates:
-  // one n = 512 solvec 403 -> 383 us, n = 16384 40.9 -> 40.3 ms), and f16
-  // operands on 128 x 128 tiles.  Measured on the SYRK
-  // at n = 32256, k = 512: f64 53 -> 57, f16 199 -> 348 TFLOP/s; on the
-  // look-ahead update as well, n = 32768: f64 solve 219.7 -> 217.4 ms, FP16+IR
-  // 81.0 -> 79.6 ms.  Not
-  // for f32 operands (88 -> 107 TFLOP/s): folding C into the f32 sum mid-way
-  // costs the accuracy that refinement then pays for (11 instead of 3 steps at
-  // cond ~4e6), and holding C to the end does not fit the registers.  Seeding
-  // the f32 accumulators with C before the first slab is no better: 119 instead
-  // of 104 TFLOP/s alone, no gain inside the factor (149.6 -> 148.4 ms at
-  // n = 32768), and 29 instead of 4 refinement steps at lambda = 1e-6.
-  constexpr bool PRE = TRI && (((BM == 256 || BM == 64) && sizeof(T) == 8) || sizeof(TI) == 2);
+  // C prefetch for the triangular updates: f64 on 64 x 64 tiles (the small blocked
+  // factors' updates: one n = 512 solvec 403 -> 383 us) and f16 operands on 128 x
+  // 128 tiles (n = 32256, k = 512: 199 -> 348 TFLOP/s).  Not for f32 operands (88 ->
+  // 107 TFLOP/s): folding C into the f32 sum mid-way costs the accuracy that
+  // refinement then pays for (11 instead of 3 steps at cond ~4e6), and holding C to
+  // the end does not fit the registers.  Seeding the f32 accumulators with C before
+  // the first slab is no better: 119 instead of 104 TFLOP/s alone, no gain inside
+  // the factor (149.6 -> 148.4 ms at n = 32768), and 29 instead of 4 refinement
+  // steps at lambda = 1e-6.
+  constexpr bool PRE = TRI && ((BM == 64 && sizeof(T) == 8) || sizeof(TI) == 2);
   nt_tile<T, BM, BN, WM, WN, TRI, VEC, PRE, TI>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, m0, n0);
+}
+
+// ---------------------------------------------------------------------------
+// C -= A B^T on 128 x 128 tiles (TRI: row >= col; SQ: the square triangular case)
+// for the large updates of the factor: operands go from global memory straight to
+// LDS (16 bytes a lane), so that no staging registers stand between a wave's
+// accumulators (64 x 64) and the register file, and two workgroups of four waves
+// share a CU: while one waits at its barrier or for its C tile, the other's MFMAs
+// run.  A slab is 128 bytes of k per row; a slab's fragments are read into
+// registers first, then the next slab's loads are issued, then the slab's MFMAs
+// run (4096 cycles a wave), which the loads have to land.
+//
+// A load writes its wave's 64 x 16 bytes to LDS in lane order, eight rows of eight
+// 16-byte pieces, so rows cannot be padded; piece v of row r is stored at v ^ (r %
+// 8) instead (the lane asks for that piece), and the 8 rows of a fragment read's
+// phase meet 8 different bank groups.
+//
+// K is a multiple of the slab, pointers and rows are 16-byte aligned (the
+// launcher's rule).  Rows beyond M (N) read the last one, and are not stored.
+//
+// What bounds it: MFMA issue.  Measured alone, C -= P P^T (lower): f64 n = 30720,
+// k = 1024 68.2 TFLOP/s (256 x 128 tiles through registers 57-62), f32 122 (128 x
+// 128 through registers 107); without the loads the same loop takes 71 and 136.
+template <typename T, bool TRI, bool SQ>
+__global__ __launch_bounds__(256, 2) void nt_dma_kernel(int M, int N, int K, const T* __restrict__ A, int64_t lda,
+                                                        const T* __restrict__ B, int64_t ldb, T* __restrict__ C,
+                                                        int64_t ldc, const int32_t* __restrict__ gate, int tiles_m,
+                                                        int tiles_n, int total) {
+  constexpr int BM = 128, NW = 4, VL = 16 / sizeof(T), SK = 8 * VL, ROW = 128;  // bytes of a slab row
+  using MF = Mfma<T>;
+  using acc_t = typename MF::acc_t;
+  typedef T vec_t __attribute__((ext_vector_type(VL)));
+  __shared__ __attribute__((aligned(1024))) char lds[2][2 * BM * ROW];
+  if (gate != nullptr && *gate != kNoFail) return;
+  const int per = (total + 7) / 8, lin = (blockIdx.x % 8) * per + blockIdx.x / 8;
+  if (lin >= total) return;
+  int tm, tn;
+  if (SQ) {
+    tri_tile(lin, tiles_m, tiles_n, 1, tm, tn);
+  } else {
+    const int per_group = kGroupM * tiles_n, g = lin / per_group, first = g * kGroupM;
+    const int gm = min(kGroupM, tiles_m - first), r = lin - g * per_group;
+    tm = first + r % gm;
+    tn = r / gm;
+  }
+  const int m0 = tm * BM, n0 = tn * BM;
+  if (TRI && m0 + BM - 1 < n0) return;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+
+  // this wave's loads: chunks of 8 rows, A's 16 then B's 16
+  constexpr int CPW = 2 * BM / 8 / NW;
+  uint32_t voff[CPW];
+#pragma unroll
+  for (int j = 0; j < CPW; ++j) {
+    const int ch = wave + NW * j;
+    const bool a = ch < BM / 8;
+    const int row = (a ? ch : ch - BM / 8) * 8 + (lane >> 3);
+    const int r = a ? min(m0 + row, M - 1) - m0 : min(n0 + row, N - 1) - n0;
+    voff[j] = (uint32_t)r * (uint32_t)((a ? lda : ldb) * sizeof(T)) + ((lane & 7) ^ (lane >> 3)) * 16;
+  }
+  const char* const pa = reinterpret_cast<const char*>(A + (int64_t)m0 * lda);
+  const char* const pb = reinterpret_cast<const char*>(B + (int64_t)n0 * ldb);
+  auto issue = [&](int s, int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < CPW; ++j) {
+      const int ch = wave + NW * j;
+      const char* src = (ch < BM / 8 ? pa : pb) + (int64_t)s * ROW + voff[j];
+      __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)src,
+                                       (__attribute__((address_space(3))) void*)&lds[buf][ch * 8 * ROW], 16, 0, 0);
+    }
+  };
+
+  acc_t acc[4][4];
+#pragma unroll
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+  const int off = (lane & 15) * ROW + ((lane >> 4) ^ (lane & 7)) * 16;
+  vec_t af[2][4], bf[2][4];
+  auto frags = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        af[c][i] = *reinterpret_cast<const vec_t*>(&lds[buf][wm * ROW + (off ^ (c * 64)) + i * 16 * ROW]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        bf[c][i] = *reinterpret_cast<const vec_t*>(&lds[buf][(BM + wn) * ROW + (off ^ (c * 64)) + i * 16 * ROW]);
+    }
+  };
+  auto mul = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+      for (int e = 0; e < VL; ++e)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[i][j] = MF::mma(af[c][i][e], bf[c][j][e], acc[i][j]);
+  };
+  // the C tile, read 16 rows of a wave at a time from indices clamped into the
+  // matrix (an entry above the diagonal is still C's memory)
+  const int ci = m0 + wm + MF::row(lane, 0), cj = n0 + wn + (lane & 15);
+  const bool inside = m0 + BM <= M && n0 + BM <= N;
+  auto cload = [&](int i, T (&v)[4][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gi = ci + 16 * i + MF::kRowStep * r, gj = cj + 16 * j;
+        v[j][r] = inside ? C[(int64_t)gi * ldc + gj] : C[(int64_t)min(gi, M - 1) * ldc + min(gj, N - 1)];
+      }
+  };
+  auto cstore = [&](int i, const T (&v)[4][4]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int gi = ci + 16 * i + MF::kRowStep * r, gj = cj + 16 * j;
+        if ((inside || (gi < M && gj < N)) && (!TRI || gj <= gi)) C[(int64_t)gi * ldc + gj] = v[j][r] - acc[i][j][r];
+      }
+  };
+
+  const int ns = K / SK;
+  issue(0, 0);
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+  __syncthreads();
+  int s = 0;
+  for (; s + 1 < ns; ++s) {
+    frags(s & 1);
+    // (the scheduler would move the wait and the barrier up among the MFMAs, which
+    // touch no memory)
+    __builtin_amdgcn_sched_barrier(0);
+    issue(s + 1, (s & 1) ^ 1);
+    __builtin_amdgcn_sched_barrier(0);
+    mul();
+    __builtin_amdgcn_sched_barrier(0);
+    __syncthreads();
+  }
+  T v0[4][4], v1[4][4];
+  frags(s & 1);
+  __builtin_amdgcn_sched_barrier(0);
+  cload(0, v0);
+  __builtin_amdgcn_sched_barrier(0);
+  mul();
+  cload(1, v1);
+  cstore(0, v0);
+  cload(2, v0);
+  cstore(1, v1);
+  cload(3, v1);
+  cstore(2, v0);
+  cstore(3, v1);
+}
+
+// Whether nt_dma_kernel takes these operands: whole slabs of k, 16-byte pieces, row
+// offsets of a tile within 32 bits.
+template <typename T>
+bool nt_dma_ok(int K, const T* A, int64_t lda, const T* B, int64_t ldb) {
+  const int64_t rb = std::max(lda, ldb) * (int64_t)sizeof(T);
+  return K > 0 && K % (128 / (int)sizeof(T)) == 0 && reinterpret_cast<uintptr_t>(A) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(B) % 16 == 0 && (lda * sizeof(T)) % 16 == 0 && (ldb * sizeof(T)) % 16 == 0 &&
+         rb < ((int64_t)1 << 24);
+}
+
+template <typename T, bool TRI, bool SQ>
+hipError_t launch_nt_dma(int M, int N, int K, const T* A, int64_t lda, const T* B, int64_t ldb, T* C, int64_t ldc,
+                         const int32_t* gate, hipStream_t s) {
+  const int tiles_m = (M + 127) / 128, tiles_n = (N + 127) / 128;
+  const int total = SQ ? tri_total(tiles_m, tiles_n, 1) : tiles_m * tiles_n;
+  hipLaunchKernelGGL((nt_dma_kernel<T, TRI, SQ>), dim3(8 * ((total + 7) / 8)), dim3(256), 0, s, M, N, K, A, lda, B,
+                     ldb, C, ldc, gate, tiles_m, tiles_n, total);
+  return hipGetLastError();
 }
 
 // SQ launches the square lower-triangle form (M == N, TRI), which only the
@@ -313,10 +483,9 @@ hipError_t launch_gemm(bool ta, bool tb, bool tri, int M, int N, int K, T alpha,
   if (M <= 0 || N <= 0) return hipSuccess;
   if (K <= 0) K = 0;
   if (!ta && tb) {
-    // Large updates: 256 x 128 tiles on 8 waves (2 per SIMD) cut the operand
-    // traffic per flop by a quarter; smaller ones keep 128 x 128 tiles so the
-    // grid still fills the 256 CUs; narrow ones (N <= 64, the panel solve) and
-    // small ones that would give fewer than 128 such tiles use 64 x 64 tiles.
+    // Large updates: 128 x 128 tiles, operands straight to LDS where they allow it
+    // (nt_dma_kernel); narrow ones (N <= 64, the panel solve) and small ones that
+    // would give fewer than 128 such tiles use 64 x 64 tiles.
     // Triangular updates enumerate the full rectangle; tiles wholly above the
     // diagonal exit at once.  A and C may alias when every tile holds all of
     // its rows' k (the in-place panel solve: N = K <= 64, one tile column).
@@ -327,18 +496,13 @@ hipError_t launch_gemm(bool ta, bool tb, bool tri, int M, int N, int K, T alpha,
       if (tri) return launch_nt<T, 64, 64, 2, 4, true>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate, s);
       return launch_nt<T, 64, 64, 2, 4, false>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate, s);
     }
-    // 256 x 128 only for f64: the f32 instantiation of that tile ran the
-    // look-ahead panel update (M = 31744, N = K = 1024) at 5.3 ms per launch
-    // against 2.0 ms for f64 on the same shapes, while 128 x 128 is the faster
-    // f32 tile for the SYRK too.
-    // 128 x 128 tiles on 16 waves, as the SYRK's (f64 solve at n = 32768 215.7
-    // -> 212.8 ms, FP32+IR 140.0 -> 136.0 ms against 4 waves).
-    const bool big = sizeof(T) == 8 && (int64_t)M * N >= (int64_t)4096 * 4096;
-    if (tri) {
-      if (big) return launch_nt<T, 256, 128, 4, 2, true>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate, s);
-      return launch_nt<T, 128, 128, 4, 4, true>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate, s);
+    if (alpha == T(-1) && beta == T(1) && nt_dma_ok<T>(K, A, lda, B, ldb)) {
+      if (tri) return launch_nt_dma<T, true, false>(M, N, K, A, lda, B, ldb, C, ldc, gate, s);
+      return launch_nt_dma<T, false, false>(M, N, K, A, lda, B, ldb, C, ldc, gate, s);
     }
-    if (big) return launch_nt<T, 256, 128, 4, 2, false>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate, s);
+    // 128 x 128 tiles on 16 waves (f64 solve at n = 32768 215.7 -> 212.8 ms, FP32+IR
+    // 140.0 -> 136.0 ms against 4 waves).
+    if (tri) return launch_nt<T, 128, 128, 4, 4, true>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate, s);
     return launch_nt<T, 128, 128, 4, 4, false>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate, s);
   }
   if (!ta && tb && tri)
@@ -357,16 +521,10 @@ hipError_t launch_syrk_lower(int n, int k, T alpha, const T* A, int64_t lda, T b
                              const int32_t* gate, hipStream_t s) {
   if (n <= 0) return hipSuccess;
   if (k < 0) k = 0;
-  // f64: 256 x 128 tiles on 8 waves (2 per SIMD) while the grid still fills the
-  // chip several times over, 128 x 128 tiles for the last few small updates.
-  // f32: 128 x 128 tiles throughout (measured faster than 256 x 128 for f32).
-  // The 128 x 128 tiles run on 16 waves (32 x 32 each, 56 VGPRs in f32, eight
-  // waves per SIMD): n = 32768 FP32+IR 148.8 -> 140.0 ms (f32 SYRK 88 -> 97
-  // TFLOP/s) against the 4-wave form; 8 waves (2 x 4 or 4 x 2) gave 142 ms,
-  // 256 x 128 on 16 waves 147 ms.  For f64, 16 waves on 256 x 128 (a 64 x 32
-  // tile per wave at 128 VGPRs) took the solve from 216 to 225 ms.
-  if (sizeof(T) == 8 && (int64_t)n * n >= (int64_t)4096 * 4096)
-    return launch_nt<T, 256, 128, 4, 2, true, true>(n, n, k, alpha, A, lda, A, lda, beta, C, ldc, gate, s);
+  // Operands that cannot go straight to LDS take 128 x 128 tiles through registers
+  // on 16 waves, the same sums in the same order.
+  if (alpha == T(-1) && beta == T(1) && nt_dma_ok<T>(k, A, lda, A, lda))
+    return launch_nt_dma<T, true, true>(n, n, k, A, lda, A, lda, C, ldc, gate, s);
   return launch_nt<T, 128, 128, 4, 4, true, true>(n, n, k, alpha, A, lda, A, lda, beta, C, ldc, gate, s);
 }
 

@@ -17,15 +17,12 @@ constexpr int32_t kNoFail = 0x7fffffff;
 // panel width, the rank of the trailing SYRK update on MFMA, is kNBO, or
 // kNBO_LARGE for an order of at least kNBO_LARGE_N when the SYRK runs on f64 or
 // f32 operands (outer_width()).  Wider panels give each output tile more MFMA
-// k-slabs per read-modify-write of C but a longer panel chain.  Measured solves:
-// n = 32768 f64 229 / 220 / 223 / 226 ms at 512 / 1024 / 1536 / 2048; n = 16384
-// f64 41.6 / 42.5 ms at 512 / 1024; the f16-operand factor, whose SYRK is fast and
+// k-slabs per read-modify-write of C but a longer panel chain.  Measured: solve n =
+// 32768 f64 194.7 / 195.9 / 198.6 ms at 1024 / 768 / 1536, FP32 refined 137.0 / 138.5 /
+// 137.8; potrf n = 16384 f64 29.5 / 29.7 ms at 512 / 1024; the f16-operand factor, whose SYRK is fast and
 // whose panel chain sets the pace, 87 / 95 ms at 512 / 1024 (n = 32768), and later
 // FP16+IR 88.5 / 78.1 / 70.8 ms at 256 / 384 / 512 (narrower panels pass over the
-// f32 trailing matrix more often); the FP32
-// refined solve 166 / 158 ms at 512 / 1024 (n = 32768: its rank-512 SYRKs cost
-// more than the shorter panel chain saves), later 134.6 / 133.4 / 134.6 ms at
-// 768 / 1024 / 1536.
+// f32 trailing matrix more often).
 constexpr int kNB = 64;
 constexpr int kNBO = 512;
 constexpr int kNBO_LARGE = 1024;
