@@ -114,8 +114,10 @@ const Lookahead* ctx_lookahead(llh_context* ctx) {
     Lookahead la;
     if (hipStreamCreateWithFlags(&la.side, hipStreamNonBlocking) != hipSuccess) return nullptr;
     if (hipEventCreateWithFlags(&la.fork, hipEventDisableTiming) != hipSuccess ||
-        hipEventCreateWithFlags(&la.join, hipEventDisableTiming) != hipSuccess) {
+        hipEventCreateWithFlags(&la.join, hipEventDisableTiming) != hipSuccess ||
+        hipEventCreateWithFlags(&la.rows, hipEventDisableTiming) != hipSuccess) {
       if (la.fork) (void)hipEventDestroy(la.fork);
+      if (la.join) (void)hipEventDestroy(la.join);
       (void)hipStreamDestroy(la.side);
       return nullptr;
     }
@@ -836,6 +838,7 @@ void llh_context_destroy(llh_context* ctx) {
     (void)hipStreamSynchronize(ctx->la.side);
     (void)hipEventDestroy(ctx->la.fork);
     (void)hipEventDestroy(ctx->la.join);
+    (void)hipEventDestroy(ctx->la.rows);
     (void)hipStreamDestroy(ctx->la.side);
     if (ctx->la.fwd) {
       (void)hipStreamSynchronize(ctx->la.fwd);

@@ -26,66 +26,39 @@ namespace llh {
 
 namespace {
 
-// Factors the outer panel of columns [k0, k0 + kb) on stream st, everything
-// left of k0 having been applied to these columns.  The panel is split in two
-// halves recursively down to kNB columns: factor the left half, update the
-// right half's columns with it (one GEMM, rank = the left half's width, lower
-// part of the top square), factor the right half.  A kNB-wide block is the
-// diagonal block in LDS (with its inverse), then the rows below it as one MFMA
-// product with that inverse.  (A panel of few rows goes by step launches instead;
-// *stepped tells whether its last block's L still waits beside its place.)  Against
-// a kNB-at-a-time right-looking sweep the
-// launches are as many, but each column of the panel is read and written by
-// log2(kb / kNB) updates instead of up to kb / kNB - 1, and the updates have rank
-// 64 .. 256 instead of 64.
+// The rows of the panel [k0, k0 + kb) that its steps factor end here.
+int top_end(int n, int k0, int kb) { return n - k0 <= kStepRows ? n : k0 + kb; }
+
+// Factors the columns [k0, k0 + kb) of the rows k0 .. n on stream st, everything left
+// of k0 having been applied to them: one launch per 64 columns.  *stepped: whether
+// the block before k0 still waits beside its place (launch_panel_step).
 template <typename T>
-hipError_t factor_panel(T* a, int64_t lda, int n, int k0, int kb, int32_t* info, T* dinv, hipStream_t st,
-                        Profiler* prof, bool diag_f64, bool* stepped) {
+hipError_t factor_steps(T* a, int64_t lda, int n, int k0, int kb, int32_t* info, T* dinv, bool beside, bool* stepped,
+                        hipStream_t st, Profiler* prof, bool diag_f64) {
   const double es = (double)sizeof(T);
-  if (n - k0 <= step_rows<T>()) {
-    for (int k = k0; k < k0 + kb; k += kNB) {
-      const double db = std::min(kNB, n - k), below = std::max(0, n - k - kNB), pb = k > k0 ? db : 0.0;
-      const double cols = std::max(0, k0 + kb - k - kNB);
-      const double outs = below * cols - cols * (cols - 1.0) / 2.0;
-      LLH_PROF_ON(st, kDiagFactor, 2.0 * db * db * db / 3.0 + 2.0 * below * db * (db + pb) + 2.0 * outs * pb,
-                  es * (2.0 * db * db + below * (2.0 * db + pb) + (pb > 0.0 ? 2.0 * outs : 0.0)),
-                  (diag_f64 && sizeof(T) == 4
-                       ? launch_panel_step<T, double>(a, lda, n, k, k0, k0 + kb, dinv, info, *stepped, st)
-                       : launch_panel_step<T>(a, lda, n, k, k0, k0 + kb, dinv, info, *stepped, st)));
-      *stepped = true;
-    }
-    return hipSuccess;
+  const int end = k0 + kb;
+  for (int k = k0; k < end; k += kNB) {
+    const double db = std::min(kNB, n - k), below = std::max(0, n - k - kNB), pb = k > k0 ? db : 0.0;
+    const double cols = std::max(0, end - k - kNB);
+    const double outs = below * cols - cols * (cols - 1.0) / 2.0;
+    LLH_PROF_ON(st, kDiagFactor, 2.0 * db * db * db / 3.0 + 2.0 * below * db * (db + pb) + 2.0 * outs * pb,
+                es * (2.0 * db * db + below * (2.0 * db + pb) + (pb > 0.0 ? 2.0 * outs : 0.0)),
+                (diag_f64 && sizeof(T) == 4
+                     ? launch_panel_step<T, double>(a, lda, n, k, k0, end, dinv, info, *stepped, beside, st)
+                     : launch_panel_step<T>(a, lda, n, k, k0, end, dinv, info, *stepped, beside, st)));
+    *stepped = k + kNB < n;
   }
-  if (kb > kNB) {
-    const int h = (kb / kNB + 1) / 2 * kNB;  // left half: a whole number of blocks, at least one
-    LLH_TRY(factor_panel<T>(a, lda, n, k0, h, info, dinv, st, prof, diag_f64, stepped));
-    const int below = n - k0 - h, cols = kb - h;  // rows k0+h.., columns k0+h .. k0+kb
-    T* left = a + (int64_t)(k0 + h) * lda + k0;    // L of rows k0+h.., columns k0 .. k0+h
-    const double outs = (double)below * cols - (double)cols * (cols - 1) / 2.0, dh = h;
-    LLH_PROF_ON(st, kPanelUpdate, 2.0 * outs * dh, es * (2.0 * outs + ((double)below + cols) * dh),
-                (launch_gemm<T>(false, true, true, below, cols, h, T(-1), left, lda, left, lda, T(1), left + h, lda,
-                                info, st)));
-    return factor_panel<T>(a, lda, n, k0 + h, cols, info, dinv, st, prof, diag_f64, stepped);
-  }
-  const int k = k0, b = kb;
-  T* akk = a + (int64_t)k * lda + k;
-  const double db = b;
-  T* dk = dinv + (int64_t)(k / kNB) * kNB * kNB;
-  if (diag_f64 && sizeof(T) == 4) {
-    LLH_PROF_ON(st, kDiagFactor, 2.0 * db * db * db / 3.0, es * db * db * 2.0,
-                (launch_diag_fast<T, double>(akk, lda, b, dk, info, k, info, st)));
-  } else {
-    LLH_PROF_ON(st, kDiagFactor, 2.0 * db * db * db / 3.0, es * db * db * 2.0,
-                (launch_diag_fast<T>(akk, lda, b, dk, info, k, info, st)));
-  }
-  const int below = n - k - b;
-  if (below <= 0) return hipSuccess;
-  T* panel = akk + (int64_t)b * lda;  // rows k+b.., columns k..k+b
-  // L21 = A21 * L11^-T as one MFMA product with the inverse, in place (each
-  // workgroup reads all of its rows' k before writing them).
-  LLH_PROF_ON(st, kPanelTrsm, (double)below * db * db * 2.0, es * ((double)below * db * 2.0 + db * db),
-              (launch_gemm<T>(false, true, false, below, b, b, T(1), panel, lda, dk, kNB, T(0), panel, lda, info,
-                              st)));
+  return hipSuccess;
+}
+
+// The rows below the factored top block of a panel: L21 = A21 L11^-T.
+template <typename T>
+hipError_t factor_rows(T* a, int64_t lda, int n, int k0, int kb, int32_t* info, const T* dinv, hipStream_t st,
+                       Profiler* prof) {
+  const double below = n - top_end(n, k0, kb), dkb = kb;
+  if (below <= 0.0) return hipSuccess;
+  LLH_PROF_ON(st, kPanelTrsm, below * dkb * dkb, sizeof(T) * (2.0 * below * dkb + dkb * dkb / 2.0),
+              (launch_panel_rows<T>(a, lda, n, k0, kb, dinv, info, st)));
   return hipSuccess;
 }
 
@@ -107,11 +80,12 @@ hipError_t trailing_syrk(int m, int kb, const T* p, int64_t lda, T* c, int32_t* 
 }  // namespace
 
 // Right-looking blocked Cholesky of the lower triangle (the blocked equivalent
-// of cholesky.rs:54-74).  Each outer panel (panel_width() columns) is factored
-// by factor_panel; then one SYRK of that rank on MFMA updates the trailing matrix.
-// With lookahead, the trailing update of panel k is split: the next panel's
-// columns are updated and that panel factored on the side stream while the SYRK
-// of the remaining trailing matrix runs on s.  Matrices no larger than the LDS
+// of cholesky.rs:54-74).  Each outer panel (panel_width() columns) is factored in
+// steps of 64 columns (factor_steps, and factor_rows for the rows that these leave);
+// then one SYRK of that rank on MFMA updates the trailing matrix.  With lookahead, the
+// trailing update of panel k is split: the rows of the next panel's steps are updated
+// and the steps taken on the side stream while s updates the panel's other rows and
+// then the remaining trailing matrix.  Matrices no larger than the LDS
 // kernel's limit are factored by that kernel alone, in the reference's exact
 // operation order.
 template <typename T>
@@ -148,8 +122,9 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
     if (dinv != nullptr) LLH_TRY(launch_trtri_blocks<T>(n, a, lda, false, false, dinv, info, s));
   } else {
     const int kb0 = std::min(panel_width(n, n, half != nullptr), n);
-    bool stepped = false;  // the last block column was a step launch (its L_kk is still beside its place)
-    LLH_TRY(factor_panel<T>(a, lda, n, 0, kb0, info, dinv, s, prof, diag_f64, &stepped));
+    bool stepped = false;
+    LLH_TRY(factor_steps<T>(a, lda, top_end(n, 0, kb0), 0, kb0, info, dinv, false, &stepped, s, prof, diag_f64));
+    LLH_TRY(factor_rows<T>(a, lda, n, 0, kb0, info, dinv, s, prof));
     if (ff != nullptr) {
       LLH_TRY(hipEventRecord(la->fwd_ev, s));
       LLH_TRY(hipStreamWaitEvent(la->fwd, la->fwd_ev, 0));
@@ -170,7 +145,9 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
         const double outs = (double)m2 * (m2 + 1) / 2.0;
         LLH_PROF(kTrailingSyrk, 2.0 * outs * kb, es * 2.0 * outs + pes * (double)m2 * kb,
                  (trailing_syrk<T>(m2, kb, p, lda, c, info, half, s)));
-        LLH_TRY(factor_panel<T>(a, lda, n, k0 + kb, kb2, info, dinv, s, prof, diag_f64, &stepped));
+        LLH_TRY(factor_steps<T>(a, lda, top_end(n, k0 + kb, kb2), k0 + kb, kb2, info, dinv, false, &stepped, s, prof,
+                                diag_f64));
+        LLH_TRY(factor_rows<T>(a, lda, n, k0 + kb, kb2, info, dinv, s, prof));
         continue;
       }
       // With half, the whole panel (m2 x kb) is rounded to f16 once, before the
@@ -184,28 +161,47 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
       }
       LLH_TRY(hipEventRecord(la->fork, s));
       LLH_TRY(hipStreamWaitEvent(la->side, la->fork, 0));
+      const int m3 = m2 - kb2;  // the rest of the trailing matrix
+      const int end2 = top_end(n, k0 + kb, kb2), mt = end2 - k0 - kb, mr = n - end2;  // next panel's rows: steps, below
       {
-        // next panel's columns (m2 rows x kb2 columns, lower part of the top
-        // square), then its factor, on the side stream
-        const double outs = (double)m2 * kb2 - (double)kb2 * (kb2 - 1) / 2.0;
+        // the rows of the next panel's steps, then these, on the side stream
+        const double outs = (double)mt * kb2 - (double)kb2 * (kb2 - 1) / 2.0;
         if (half_ready) {
           if constexpr (sizeof(T) == 4)
-            LLH_PROF_ON(la->side, kPanelUpdate, 2.0 * outs * kb, 4.0 * 2.0 * outs + 2.0 * ((double)m2 + kb2) * kb,
-                        (launch_gemm_nt_tri_h(m2, kb2, kb, -1.0f, half, kb, half, kb, 1.0f, c, lda, info,
-                                              la->side)));
+            LLH_PROF_ON(la->side, kPanelUpdate, 2.0 * outs * kb, 4.0 * 2.0 * outs + 2.0 * (double)mt * kb,
+                        (launch_gemm_nt_h(true, mt, kb2, kb, -1.0f, half, kb, half, kb, 1.0f, c, lda, info,
+                                          la->side)));
         } else {
-          LLH_PROF_ON(la->side, kPanelUpdate, 2.0 * outs * kb, es * (2.0 * outs + ((double)m2 + kb2) * kb),
-                      (launch_gemm<T>(false, true, true, m2, kb2, kb, T(-1), p, lda, p, lda, T(1), c, lda, info,
+          LLH_PROF_ON(la->side, kPanelUpdate, 2.0 * outs * kb, es * (2.0 * outs + (double)mt * kb),
+                      (launch_gemm<T>(false, true, true, mt, kb2, kb, T(-1), p, lda, p, lda, T(1), c, lda, info,
                                       la->side)));
         }
-        LLH_TRY(factor_panel<T>(a, lda, n, k0 + kb, kb2, info, dinv, la->side, prof, diag_f64, &stepped));
+        LLH_TRY(factor_steps<T>(a, lda, end2, k0 + kb, kb2, info, dinv, (mr > 0), &stepped, la->side, prof,
+                                diag_f64));
+      }
+      if (mr > 0) {
+        // its rows below, on s; then their solve, on the side stream
+        const double outs = (double)mr * kb2;
+        T* c2 = c + (int64_t)kb2 * lda;
+        if (half_ready) {
+          if constexpr (sizeof(T) == 4)
+            LLH_PROF(kPanelUpdate, 2.0 * outs * kb, 4.0 * 2.0 * outs + 2.0 * ((double)mr + kb2) * kb,
+                     (launch_gemm_nt_h(false, mr, kb2, kb, -1.0f, half + (int64_t)kb2 * kb, kb, half, kb, 1.0f, c2,
+                                       lda, info, s)));
+        } else {
+          LLH_PROF(kPanelUpdate, 2.0 * outs * kb, es * (2.0 * outs + ((double)mr + kb2) * kb),
+                   (launch_gemm<T>(false, true, false, mr, kb2, kb, T(-1), p + (int64_t)kb2 * lda, lda, p, lda, T(1),
+                                   c2, lda, info, s)));
+        }
+        LLH_TRY(hipEventRecord(la->rows, s));
+        LLH_TRY(hipStreamWaitEvent(la->side, la->rows, 0));
+        LLH_TRY(factor_rows<T>(a, lda, n, k0 + kb, kb2, info, dinv, la->side, prof));
       }
       LLH_TRY(hipEventRecord(la->join, la->side));
       if (ff != nullptr) {
         LLH_TRY(hipStreamWaitEvent(la->fwd, la->join, 0));
         LLH_TRY(fwd_panel(k0 + kb, kb2));
       }
-      const int m3 = m2 - kb2;  // the rest of the trailing matrix
       if (m3 > 0) {
         const double outs = (double)m3 * (m3 + 1) / 2.0;
         T* p3 = p + (int64_t)kb2 * lda;

@@ -1,24 +1,11 @@
-// Fast factor + inverse of one 64 x 64 diagonal block for the blocked paths
-// (the device code is in k_diag_impl.h): one workgroup per block, or per
-// (system, block) of a grouped batch step.
+// Fast factor + inverse of 64 x 64 diagonal blocks (the device code is in
+// k_diag_impl.h) for a grouped batch step: one workgroup per (system, block).
 #include "k_diag_impl.h"
 #include "k_subst_impl.h"
 #include "llh_kernels.h"
 
 namespace llh {
 namespace {
-
-template <typename TS, typename T>
-__global__ __launch_bounds__(kDiagT) void diag_fast_kernel(TS* __restrict__ a, int64_t lda, int b,
-                                                           TS* __restrict__ inv, int32_t* __restrict__ info,
-                                                           int64_t info_base, const int32_t* __restrict__ gate) {
-  __shared__ __attribute__((aligned(16))) DiagLds<T> sm;
-  // the gate is read once and shared, so all four waves leave or stay together
-  if (threadIdx.x == 0) sm.skip = gate != nullptr && *gate != kNoFail;
-  __syncthreads();
-  if (sm.skip) return;
-  diag_quad_block<TS, T>(a, lda, b, inv, info, info_base, sm);
-}
 
 // Grouped form for the batch planner: work w = (item, k0) factors and inverts
 // the block at (k0, k0) of its system; a failure sets the system's status.
@@ -65,22 +52,5 @@ template hipError_t launch_grp_diag_fast<double>(const BatchBase<double>*, const
                                                  int, hipStream_t);
 template hipError_t launch_grp_diag_fast<float>(const BatchBase<float>*, const BatchItem*, const StepWork*, int,
                                                 hipStream_t);
-
-template <typename TS, typename T>
-hipError_t launch_diag_fast(TS* a, int64_t lda, int b, TS* inv, int32_t* info, int64_t info_base,
-                            const int32_t* gate, hipStream_t s) {
-  if (b <= 0) return hipSuccess;
-  if (b > kNB) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((diag_fast_kernel<TS, T>), dim3(1), dim3(kDiagT), 0, s, a, lda, b, inv, info, info_base,
-                     gate);
-  return hipGetLastError();
-}
-
-template hipError_t launch_diag_fast<double, double>(double*, int64_t, int, double*, int32_t*, int64_t,
-                                                     const int32_t*, hipStream_t);
-template hipError_t launch_diag_fast<float, float>(float*, int64_t, int, float*, int32_t*, int64_t,
-                                                   const int32_t*, hipStream_t);
-template hipError_t launch_diag_fast<float, double>(float*, int64_t, int, float*, int32_t*, int64_t,
-                                                    const int32_t*, hipStream_t);
 
 }  // namespace llh

@@ -216,7 +216,7 @@ template <typename T>
 constexpr int diag_blk() { return kDiagW * diag_ls<T>(); }
 
 // 38.1 KB in f64 (four workgroups per CU).  Inside diag_quad_block l holds 14
-// blocks: the published strips (4), the sweep's results (2 x 4) and L_ww (2); a
+// blocks: the steps' strips, published and then swept (3 x 4), and L_ww (2); a
 // caller may use l and x as scratch afterwards.
 template <typename T>
 struct DiagLds {
@@ -227,34 +227,33 @@ struct DiagLds {
   int skip;                // the system has already failed: nothing to do
 };
 
-// The four steps on a 64 x 64 block whose strips are in acc (negated, see above;
-// waves wv < 4, one strip each).  Further waves of the workgroup (wv >= 4) call
-// help(w) beside sweep w, when the rows of step w - 1 are complete in the buffer
-// diag_rows(l, w - 1).  put(w, it, f) stores piece it of step w: the rows of strip
-// it (0..3) or L_ww (4), up to a failure at row f (f < 0: none).  Returns the
-// failing row or -1, the same in every thread.  l: 14 * diag_blk<T>() elements of
-// LDS, fails: one word per step.  pend(w, x) runs beside sweep w on the factor waves
-// g > w and may still change their block (g, w + 1), which is x.
+// The four steps on a 64 x 64 block whose strips are in acc (negated, see above; one
+// strip per wave g).  A step's column block is published in the buffer that its
+// rows go to afterwards, and there are three such buffers: the rows of step w stay
+// until step w + 3.  put(w, it, f) stores piece it of step w: the rows of strip it
+// (0..3) or L_ww (4), up to a failure at row f (f < 0: none).  pend(w, x) runs beside
+// sweep w on the waves g > w and may still change their block (g, w + 1), which is x;
+// help(w) follows on every wave g != w, which wave w + 1 should leave early; with WIDE
+// it runs on four further waves instead, beside every sweep.  Returns
+// the failing row or -1, the same in every thread.  l: 14 * diag_blk<T>() elements
+// of LDS, fails: one word per step.
 template <typename T>
 __device__ __forceinline__ T* diag_rows(T* l, int w) {
-  return l + (4 + (w & 1) * 4) * diag_blk<T>();
+  return l + (w == 3 ? 0 : w) * 4 * diag_blk<T>();
 }
 template <typename T>
 __device__ __forceinline__ T* diag_lww(T* l, int w) {
   return l + (12 + (w & 1)) * diag_blk<T>();
 }
 
-template <typename T, typename Put, typename Help, typename Pend>
-__device__ __forceinline__ int diag_core(typename Mfma<T>::acc_t (&acc)[kNB / kDiagW], int wv, T* l, int* fails,
+template <typename T, bool WIDE = false, typename Put, typename Help, typename Pend>
+__device__ __forceinline__ int diag_core(typename Mfma<T>::acc_t (&acc)[kNB / kDiagW], int g, T* l, int* fails,
                                          Put&& put, Help&& help, Pend&& pend) {
   constexpr int W = kDiagW, NS = kNB / W, LS = diag_ls<T>(), BLK = diag_blk<T>(), VL = 16 / sizeof(T);
   using MF = Mfma<T>;
   using acc_t = typename MF::acc_t;
   typedef T vec_t __attribute__((ext_vector_type(VL)));
-  const bool factor = wv < NS;  // wave-uniform (wv comes from readfirstlane)
-  const int g = wv;
-  T* const stg = l;  // published column blocks, one per strip
-
+  const bool factor = !WIDE || g < NS;  // wave-uniform (g comes from readfirstlane)
   int fail = -1;
   // One copy of the step's code for all four steps (a quarter of the
   // instruction fetches).
@@ -273,6 +272,7 @@ __device__ __forceinline__ int diag_core(typename Mfma<T>::acc_t (&acc)[kNB / kD
     };
     // acc[0] is column block w: the blocks move down by one each step, so that the
     // registers are addressed by constants
+    T* const stg = diag_rows(l, w);
     if (factor) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) stg[g * BLK + MF::row(lane, r) * LS + fr] = -acc[0][r];
@@ -333,7 +333,7 @@ __device__ __forceinline__ int diag_core(typename Mfma<T>::acc_t (&acc)[kNB / kD
       }
       if (lane == 0) fails[w] = fm != 0 ? W * w + __builtin_ctz(fm) : -1;
     } else {
-      // meanwhile the other factor waves: the previous step's products for the
+      // meanwhile the other waves: the previous step's products for the
       // later column blocks, and its stores
       if (g > w) pend(w, acc[1]);
       if (w > 0) {
@@ -346,6 +346,7 @@ __device__ __forceinline__ int diag_core(typename Mfma<T>::acc_t (&acc)[kNB / kD
         put(w - 1, k, -1);
         if (k + 3 <= NS) put(w - 1, k + 3, -1);
       }
+      if constexpr (!WIDE) help(w);
     }
     diag_barrier();
     fail = fails[w];

@@ -253,7 +253,7 @@ __global__ __launch_bounds__(WM* WN * 64, (512 / (WM * WN * 64)) > 0 ? 512 / (WM
   // the first slab is no better: 119 instead of 104 TFLOP/s alone, no gain inside
   // the factor (149.6 -> 148.4 ms at n = 32768), and 29 instead of 4 refinement
   // steps at lambda = 1e-6.
-  constexpr bool PRE = TRI && ((BM == 64 && sizeof(T) == 8) || sizeof(TI) == 2);
+  constexpr bool PRE = (TRI && BM == 64 && sizeof(T) == 8) || sizeof(TI) == 2;
   nt_tile<T, BM, BN, WM, WN, TRI, VEC, PRE, TI>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, m0, n0);
 }
 
@@ -543,17 +543,24 @@ hipError_t launch_syrk_lower_h(int n, int k, float alpha, const _Float16* A, int
                                                                 s);
 }
 
-hipError_t launch_gemm_nt_tri_h(int M, int N, int K, float alpha, const _Float16* A, int64_t lda,
-                                const _Float16* B, int64_t ldb, float beta, float* C, int64_t ldc,
-                                const int32_t* gate, hipStream_t s) {
+hipError_t launch_gemm_nt_h(bool tri, int M, int N, int K, float alpha, const _Float16* A, int64_t lda,
+                            const _Float16* B, int64_t ldb, float beta, float* C, int64_t ldc, const int32_t* gate,
+                            hipStream_t s) {
   if (M <= 0 || N <= 0) return hipSuccess;
   if (K < 0) K = 0;
   const int64_t t128 = (int64_t)((M + 127) / 128) * ((N + 127) / 128);
-  if (N <= 64 || t128 < 128)
-    return launch_nt<float, 64, 64, 2, 2, true, false, _Float16>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate,
-                                                                  s);
-  return launch_nt<float, 128, 128, 2, 2, true, false, _Float16>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate,
-                                                                  s);
+  if (N <= 64 || t128 < 128) {
+    if (tri)
+      return launch_nt<float, 64, 64, 2, 2, true, false, _Float16>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate,
+                                                                    s);
+    return launch_nt<float, 64, 64, 2, 2, false, false, _Float16>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate,
+                                                                   s);
+  }
+  if (tri)
+    return launch_nt<float, 128, 128, 2, 2, true, false, _Float16>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate,
+                                                                    s);
+  return launch_nt<float, 128, 128, 2, 4, false, false, _Float16>(M, N, K, alpha, A, lda, B, ldb, beta, C, ldc, gate,
+                                                                   s);
 }
 
 template hipError_t launch_syrk_lower<double>(int, int, double, const double*, int64_t, double, double*, int64_t,

@@ -36,15 +36,16 @@ inline int outer_width(int n, bool half_syrk) { return (!half_syrk && n >= kNBO_
 constexpr int kStepTail = 4096;
 inline int panel_width(int rem, int n, bool half_syrk) { return rem <= kStepTail ? rem : outer_width(n, half_syrk); }
 
-// A panel whose rows number at most step_rows is factored by one launch per 64
-// columns (launch_panel_step), in which every workgroup repeats the diagonal
-// block; with more rows than that the repeated work and its rank-64 updates take
-// more from the trailing SYRK beside them than the shorter chain gives.  Measured (potrf, ms)
-// with bounds of 0 / 4096 / 8192 / 16384 rows (512-wide panels): f64 n = 8192 7.2 / 6.6 /
-// 6.2, 16384 32.7 / 32.0 / 31.5 / 31.9; f32 n = 12000 10.3 / 9.7 / 9.1 / 8.8, 16384
-// 19.7 / 19.0 / 18.5 / 18.3.
-template <typename T>
-constexpr int step_rows() { return sizeof(T) == 8 ? 8192 : 16384; }
+// A panel of at most so many rows is stepped through with all of them: every step's
+// launch solves the rows below as well.  With more, the steps take the panel's top
+// block alone, beside the trailing update, and the rows below follow in one launch:
+// the repeated work and the rank-64 updates of many rows would take more from the
+// trailing update than the shorter chain gives.  Measured (potrf, ms) with bounds of
+// 0 / 6144 / 8192 / 12288 rows: f64 n = 6000 3.50 / 3.28 / 3.28 / 3.29, 8192 6.18 / 5.98 /
+// 5.81 / 5.81, 12000 13.7 / 13.6 / 13.5 / 13.5, 20000 50.2 / 50.3 / 50.0 / 50.1; f32
+// n = 8192 4.00 / 3.92 / 3.87 / 3.88, 12000 8.43 / 8.45 / 8.40 / 8.55, 16384 17.5 / 17.4 /
+// 17.4 / 17.7.
+constexpr int kStepRows = 8192;
 
 // Right-hand-side columns per workgroup of the one-launch triangular solve, and
 // the bound on its flag waits (2^22 polls: well over 0.1 s, far above any real wait).

@@ -30,12 +30,13 @@ hipError_t solve_sync_begin(const SolveSync& sync, hipStream_t s);
 // Number of elements of the diagonal-block inverse buffer for order n.
 inline int64_t dinv_elems(int n) { return (int64_t)((n + kNB - 1) / kNB) * kNB * kNB; }
 
-// Second stream and a fork/join event pair for the factor's lookahead: while
-// the trailing SYRK of outer panel k runs on the caller's stream, the next
-// panel's columns are updated and factored on `side`.  All default priority.
+// Second stream and its events for the factor's lookahead: while the updates of
+// outer panel k run on the caller's stream, the next panel's top block is updated
+// and factored on `side`, and then, once its rows below are updated (`rows`), they
+// are solved there.  All default priority.
 struct Lookahead {
   hipStream_t side = nullptr;
-  hipEvent_t fork = nullptr, join = nullptr;
+  hipEvent_t fork = nullptr, join = nullptr, rows = nullptr;
   // third stream and its event: the forward substitution fused into the factor
   hipStream_t fwd = nullptr;
   hipEvent_t fwd_ev = nullptr;

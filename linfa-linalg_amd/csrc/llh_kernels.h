@@ -142,21 +142,21 @@ hipError_t launch_med(const BatchBase<T>* base, const BatchItem* items, int coun
 template <typename T>
 int med_resident_per_cu(bool solve);
 
-// k_diag.hip: fast factor of one b x b (b <= 64) diagonal block in place, and
-// its inverse into inv (64 x 64 row-major); a failure at block row f sets
-// *info = min(*info, info_base + f).
-template <typename TS, typename T = TS>
-hipError_t launch_diag_fast(TS* a, int64_t lda, int b, TS* inv, int32_t* info, int64_t info_base,
-                            const int32_t* gate, hipStream_t s);
-// k_step.hip: block column k0 of the panel [p0, kend) in one launch: column k0 - 64
-// applied to columns [k0, kend) (k0 > p0), the diagonal block factored and
-// inverted (dinv: the inverses of all blocks), and the rows below multiplied by
-// that inverse.  L of the diagonal block waits in the next block's slot of dinv
-// for the next launch, which puts it in its place when copy_prev is set (set it
-// on every launch but the first of a sequence).
+// k_step.hip: block column k0 of the panel of columns [p0, kend) (rows to n) in one
+// launch: column k0 - 64 applied to columns k0 .. kend (k0 > p0), the diagonal block
+// factored and inverted (dinv: the inverses of all blocks), and the rows below
+// multiplied by that inverse.  Where there are rows below, L of the diagonal block
+// waits in the next block's slot of dinv for the launch of the next block column,
+// which puts it in its place (copy_prev: it has one to put there).
+// beside: in the form that shares a CU with a workgroup of the trailing update.
 template <typename TS, typename T = TS>
 hipError_t launch_panel_step(TS* a, int64_t lda, int n, int k0, int p0, int kend, TS* dinv, int32_t* info,
-                             bool copy_prev, hipStream_t s);
+                             bool copy_prev, bool beside, hipStream_t s);
+// k_step.hip: L21 = A21 L11^-T for the rows below the factored top block [k0, k0 +
+// kb) of a panel.
+template <typename T>
+hipError_t launch_panel_rows(T* a, int64_t lda, int n, int k0, int kb, const T* dinv, const int32_t* gate,
+                             hipStream_t s);
 // k_diag.hip: grouped form over step work (factor + inverse of each block).
 template <typename T>
 hipError_t launch_grp_diag_fast(const BatchBase<T>* base, const BatchItem* items, const StepWork* work,
@@ -200,7 +200,7 @@ hipError_t launch_syrk_lower_h(int n, int k, float alpha, const _Float16* A, int
                                int64_t ldc, const int32_t* gate, hipStream_t s, int variant = 0);
 // C (M x N, f32, lower part of the top N x N square only) = beta C + alpha A B^T
 // with f16 operands: the look-ahead panel's update of the same factor.
-hipError_t launch_gemm_nt_tri_h(int M, int N, int K, float alpha, const _Float16* A, int64_t lda,
+hipError_t launch_gemm_nt_h(bool tri, int M, int N, int K, float alpha, const _Float16* A, int64_t lda,
                                 const _Float16* B, int64_t ldb, float beta, float* C, int64_t ldc,
                                 const int32_t* gate, hipStream_t s);
 
