@@ -223,7 +223,7 @@ LLH_DEV_DECL(float, s)
  * GPU's array and the array keeps the last call's contents: calls that overlap
  * on one GPU (from any context or thread) race and must be serialized by the
  * caller. */
-#define LLH_NOALLOC_SCRATCH_BYTES (16u * 1024u * 1024u + 16u * 1024u)
+#define LLH_NOALLOC_SCRATCH_BYTES (16u * 1024u * 1024u + 544u * 1024u)
 #define LLH_NOALLOC_MAX_N 16384
 llh_status llh_dev_solvec_noalloc_d(llh_context* ctx, size_t n, double* a, size_t lda, size_t m, double* b,
                                     size_t ldb, llh_error* err);

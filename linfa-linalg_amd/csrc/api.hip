@@ -145,8 +145,17 @@ hipError_t ctx_sync(llh_context* ctx, int n, int m, SolveSync* sync) {
     e = launch_fill_i32(static_cast<int32_t*>(ctx->sync.ptr), 0, (int64_t)(ctx->sync.bytes / sizeof(int32_t)),
                         ctx->stream);
     if (e != hipSuccess) return e;
-    ctx->epoch = 1;
   }
+  const int64_t chunks = std::min<int64_t>(std::max<int64_t>(nq, 1), kMailChunks);
+  e = grow(ctx, ctx->mail, (size_t)solve_mail_words(chunks) * sizeof(uint64_t), &fresh);
+  if (e != hipSuccess) return e;
+  if (fresh) {
+    e = launch_fill_i32(static_cast<int32_t*>(ctx->mail.ptr), 0, (int64_t)(ctx->mail.bytes / sizeof(int32_t)),
+                        ctx->stream);
+    if (e != hipSuccess) return e;
+  }
+  sync->mail = static_cast<uint64_t*>(ctx->mail.ptr);
+  sync->nmail = (int64_t)(ctx->mail.bytes / sizeof(uint64_t)) / solve_mail_words(1);
   sync->words = static_cast<int32_t*>(ctx->sync.ptr);
   sync->nflags = (int64_t)(ctx->sync.bytes / sizeof(int32_t)) - 2;
   sync->epoch = &ctx->epoch;
@@ -829,6 +838,7 @@ void llh_context_destroy(llh_context* ctx) {
   if (ctx->mixed_scale.ptr) (void)hipFree(ctx->mixed_scale.ptr);
   if (ctx->half_panel.ptr) (void)hipFree(ctx->half_panel.ptr);
   if (ctx->sync.ptr) (void)hipFree(ctx->sync.ptr);
+  if (ctx->mail.ptr) (void)hipFree(ctx->mail.ptr);
   if (ctx->fwd_y.ptr) (void)hipFree(ctx->fwd_y.ptr);
   for (auto& b : ctx->host_stage)
     if (b.ptr) (void)hipHostFree(b.ptr);

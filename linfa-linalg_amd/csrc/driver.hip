@@ -238,11 +238,18 @@ hipError_t trsm_split(bool upper_op, bool trans, int n, const T* a, int64_t lda,
   const double es = (double)sizeof(T);
   if (n <= solve_split<T>(m)) {
     // the launcher resets the ticket; the error word is the call's (solve_sync_begin)
-    const int32_t epoch = (*sync->epoch)++;
-    const double fl = (double)n * n * m;
-    LLH_PROF(kSolveGemm, fl, es * ((double)n * n / 2.0 + 2.0 * n * m),
-             (launch_trsm_persistent<T>(n, m, a, lda, trans, !upper_op, dinv, dinv_t, b, ldb, sync->words,
-                                        sync->words + 2, epoch, sync->words + 1, sync->spin_limit, gate, s)));
+    const int most = (int)std::min<int64_t>(sync->nmail * kSolveChunkHost, INT_MAX);
+    for (int c = 0; c < m; c += most) {
+      const int mc = std::min(most, m - c);
+      const int32_t epoch = *sync->epoch;
+      *sync->epoch += solve_epochs(n);
+      const double fl = (double)n * n * mc;
+      LLH_PROF(kSolveGemm, fl, es * ((double)n * n / 2.0 + 2.0 * n * mc),
+               (launch_trsm_persistent<T>(n, mc, a, lda, trans, !upper_op, dinv, dinv_t, b + c, ldb, sync->words,
+                                          sync->words + 2, sync->mail, epoch, sync->words + 1, sync->spin_limit,
+                                          gate, s)));
+      if (m - c <= most) break;
+    }
     return hipSuccess;
   }
   const int n1 = ((n + kNB - 1) / kNB + 1) / 2 * kNB, n2 = n - n1;
@@ -277,6 +284,7 @@ hipError_t trsm_enqueue(bool upper_op, bool trans, int n, const T* a, int64_t ld
   if (n <= 0 || m <= 0) return hipSuccess;
   const double es = (double)sizeof(T);
   if (sync != nullptr && sync->epoch != nullptr && m <= kSolveMaxCols && sync->nflags >= solve_flags<T>(n, m) &&
+      sync->mail != nullptr && sync->nmail > 0 &&
       (dinv != nullptr || (dinv_work != nullptr && (m <= 64 || sync->wild != nullptr)))) {
     if (dinv == nullptr) {
       // Above 64 columns the caller looks at *wild afterwards and, where a
@@ -329,17 +337,21 @@ hipError_t trsm_enqueue(bool upper_op, bool trans, int n, const T* a, int64_t ld
 
 // The forward and back substitution with the factor L (lower triangle of a)
 // and the inverses of its diagonal blocks (dinv, as the factor leaves them).
-// Up to kSolvePairLdsMaxN rows and kSolveCols right-hand sides it is one
-// single-workgroup launch with B in LDS and L streamed through registers
-// (launch_solve_lds), otherwise the two one-launch triangles (trsm_enqueue),
-// whose flag hops cost ~7 us per 64 rows.  For n = 512 and one right-hand side
-// the one-workgroup launch takes 68 us against 2 x 57 us for the triangles.
-constexpr int kSolvePairLdsMaxN = kSolveLdsMaxN;
+// A small one (solve_in_lds) is one single-workgroup launch with B in LDS and L
+// streamed through registers (launch_solve_lds), otherwise the two one-launch
+// triangles (trsm_enqueue).
+//
+// The one workgroup's time grows with n and m, the triangles' by a hop per 64 rows
+// only.  Factor and solve, f64, one workgroup / triangles (us): n = 200 m = 1 112 / 133, m = 4
+// 125 / 132, m = 8 140 / 132; n = 300 138 / 154, 158 / 153, 182 / 154; n = 400 203 / 200, 239 /
+// 200, 284 / 201; n = 512 m = 1 239 / 225; f32 the same within 32 rows.
+inline bool solve_in_lds(int n, int m) { return n + 32 * m <= 432 && m <= kSolveCols; }
+static_assert(432 <= kSolveLdsMaxN, "the one-workgroup solve takes them");
 template <typename T>
 hipError_t solve_pair_enqueue(int n, const T* a, int64_t lda, int m, T* b, int64_t ldb, const T* dinv,
                               SolveSync* sync, hipStream_t s, Profiler* prof, const int32_t* gate) {
   const double es = (double)sizeof(T);
-  if (n <= kSolvePairLdsMaxN && m <= kSolveCols && dinv != nullptr && lda <= INT32_MAX) {
+  if (solve_in_lds(n, m) && dinv != nullptr && lda <= INT32_MAX) {
     LLH_PROF(kSolveGemm, 2.0 * n * n * m, es * ((double)n * n + 2.0 * n * m),
              (launch_solve_lds<T>(n, m, a, lda, dinv, b, ldb, gate, s)));
     return hipSuccess;
@@ -350,7 +362,7 @@ hipError_t solve_pair_enqueue(int n, const T* a, int64_t lda, int m, T* b, int64
 
 template <typename T>
 bool forward_fusable(int n, int m, const Lookahead* la) {
-  return m > 0 && m <= 64 && n > panel_width(n, n, false) && n > kSolvePairLdsMaxN && n > small_max<T>() &&
+  return m > 0 && m <= 64 && n > panel_width(n, n, false) && n > kSolveLdsMaxN && n > small_max<T>() &&
          la != nullptr && la->fwd != nullptr && la->fwd_ev != nullptr;
 }
 

@@ -14,6 +14,7 @@
 // the column), restricted to b <= 64 rows.
 #include "llh_common.h"
 #include "llh_kernels.h"
+#include "k_gemm_impl.h"
 #include "k_trsm_impl.h"
 
 namespace llh {
@@ -162,279 +163,362 @@ __global__ __launch_bounds__(256) void trtri64_kernel(int n, const TS* __restric
 // q).  Position p is block row w = p (forward, op(A) lower) or w = nb-1-p
 // (backward).  The workgroup accumulates sum_j op(A)_wj X_j over the blocks j
 // that precede w in solve order, then forms X_w = inv(op(A)_ww) (B_w - sum) with
-// the precomputed inverse, stores it and raises flag (w, q).  A workgroup only
-// ever waits for positions taken before its own, so the chain always advances
-// whatever the residency.  Flags hold the epoch of the call that raised them, so
-// they never need clearing.
+// the precomputed inverse and publishes it.  A workgroup only ever waits for
+// positions taken before its own, so the chain always advances whatever the
+// residency.
 //
-// The walk is throughput-bound for every workgroup behind the frontier, so it
-// keeps synchronisation off the per-block path: wave v owns columns
-// [16v, 16v + 16) of each 64 x 64 tile, and each lane (row r) holds its 16 tile
-// values in registers, loaded from global memory one block ahead; X_j goes
-// through a double-buffered LDS slab with one barrier per block; and flags are
-// checked in windows: one poll and one acquire fence cover every block whose
-// flag is already raised.  The wave partial sums are reduced once.
-//
-// Only the last dependencies lie on the chain from flag to flag, so the
-// workgroup does everything else before it waits for them.  With l1 and l2 the
+// What bounds it: the chain of nb hops.  Only the last dependencies lie on it, so
+// the workgroup does everything else before it waits for them.  With l1 and l2 the
 // blocks solved just before w (l1 last), it forms at the start
-// G_i = inv(op(A)_ww) op(A)_w,li (in LDS) and B_w; after the other blocks,
-// Z = inv(op(A)_ww) (B_w - sum_{j != l1, l2} op(A)_wj X_j); once X_l2 is
-// published Z -= G_2 X_l2, and once X_l1 is, X_w = Z - G_1 X_l1.  So a flag is
-// followed by one 64 x 64 product and one reduction before the next is raised,
-// and the rest of the block's work overlaps the two steps before it.
+// G_i = inv(op(A)_ww) op(A)_w,li (in registers, as MFMA operands); after the other
+// blocks, Z = inv(op(A)_ww) (B_w - sum_{j != l1, l2} op(A)_wj X_j); then Z -= G_2 X_l2
+// and X_w = Z - G_1 X_l1.  A hop is then one transfer between CUs and one 64 x 64 x 16
+// product on MFMA, 16 rows a wave, without a reduction.
+//
+// The transfer is one store and one load: each 32-bit half of X_w travels in a 64-bit
+// word beside a tag of the call and position (relaxed atomics of agent scope, which
+// go past the L2s), so a reader polls the data itself instead of a flag, and neither
+// side needs a fence (a release writes the whole L2 back, an acquire drops it).  The
+// words lie in a ring of kMailRing blocks a chunk.  Only the kMailReach positions after
+// a block read it there, and a position publishes after it has read its own
+// dependencies, so a block's slot is free once its successor kMailRing later is
+// reached (kMailReach < kMailRing).  Positions further behind read B itself, once the
+// block's flag, raised after its stores have reached memory, holds the call's epoch.
+//
+// The walk over the other blocks is split by k: wave v multiplies columns
+// [16 v, 16 v + 16) of each tile for all 64 rows, with both operands loaded straight
+// into registers (tiles one block ahead), and polls for itself, so it has no barrier;
+// the wave partial sums are reduced once.
+//
+// Against one flag per block between fences, with the products on the VALU (us a
+// hop, n = 12000 and m = 16): f64 6.7 -> 2.8, f32 5.0 -> 2.0; whole solves (us): n = 4096,
+// m = 64 f64 507 -> 195, f32 431 -> 156; n = 4096, m = 300 f32 599 -> 286.
+//
 // The wait is bounded: past spin_limit polls (or once another workgroup has
-// given up) the workgroup records an error and returns without raising its flag.
+// given up) the workgroup records an error and returns without publishing.
 // A negative spin_limit makes every wait give up at once (a host-forced failure
 // for tests of the error path; every workgroup still exits normally).  With a
 // gate (the factor's status word) that holds a failed row, every workgroup
 // returns at once and B is left untouched.
 constexpr int kSolveChunk = kSolveChunkHost;
 constexpr int kFlagWindow = 64;  // flags checked ahead per wait
+constexpr int kMailReach = 4;    // positions that read a block from the ring
+static_assert(kMailReach < kMailRing, "a slot's readers have published before it is written again");
+static_assert(kMailSlot >= 2 * kNB * kSolveChunkHost, "a block's words fit its slot");
 
-// f64: the three 64 x 64 tiles and the work area take 139 KB of LDS, one
-// workgroup per CU; f32: two.
+// Relaxed loads and stores of agent scope, on the value's bits.
+template <typename T>
+__device__ __forceinline__ T agent_load(const T* p) {
+  if constexpr (sizeof(T) == 8)
+    return __builtin_bit_cast(T, __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT));
+  else
+    return __builtin_bit_cast(T, __hip_atomic_load(reinterpret_cast<const uint32_t*>(p), __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT));
+}
+template <typename T>
+__device__ __forceinline__ void agent_store(T* p, T v) {
+  if constexpr (sizeof(T) == 8)
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+  else
+    __hip_atomic_store(reinterpret_cast<uint32_t*>(p), __builtin_bit_cast(uint32_t, v), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_AGENT);
+}
+
 template <typename T, bool VEC>
-__global__ __launch_bounds__(256, sizeof(T) == 8 ? 1 : 2) void trsm_persistent_kernel(
+__global__ __launch_bounds__(256, 2) void trsm_persistent_kernel(
     int n, int m, const T* __restrict__ A, int64_t lda, bool trans, bool lower_op, const T* __restrict__ Dinv,
-    bool dinv_t, T* B, int64_t ldb, int32_t* ticket, int32_t* flags, int32_t epoch, int32_t* err,
+    bool dinv_t, T* B, int64_t ldb, int32_t* ticket, int32_t* flags, uint64_t* mail, int32_t epoch, int32_t* err,
     int64_t spin_limit, const int32_t* __restrict__ gate) {
   if (gate != nullptr && *gate != kNoFail) return;
-  constexpr int MC = kSolveChunk, KW = kNB / 4, S = kNB + 1, SL = kNB * MC;
-  static_assert(MC == 16 && KW == 16, "one 16-column chunk, 16 tile columns per wave");
-  static_assert(5 * SL >= kNB * S, "a staged tile fits the work area");
-  // Work area, by phase: a staged tile of op(A) (64 x S) for G; the
-  // double-buffered X_j slabs [0, 2 SL) of the walk; the 4 wave partials
-  // [0, 4 SL) and one slab [4 SL, 5 SL) of the reductions.
-  __shared__ __attribute__((aligned(16))) T Wk[5 * SL];
-  __shared__ T Dl[kNB * S];              // inv(op(A)_ww)
-  __shared__ T Gs[2][kNB * S];           // G_1, G_2
-  __shared__ int s_ticket, s_ready, s_abort;
-  T* const Part = Wk;
-  T* const Slab = Wk + 4 * SL;
-  const int tid = threadIdx.x;
+  using MF = Mfma<T>;
+  using acc_t = typename MF::acc_t;
+  // kFar (f64): G_2 waits in LDS, since with both in registers some are spilled (3.6 us
+  // a hop instead of 2.9; one workgroup per CU instead: 476 us for 416 at n = 4096, m = 300)
+  constexpr bool kFar = sizeof(T) == 8;
+  // a slab's row k, column c is at sidx(k, c); in f32 rows 4 apart go to different banks
+  constexpr int MC = kSolveChunk, S = kNB + 1, PAD = kFar ? 0 : MC, SL = kNB * MC + kNB / 4 * PAD, NK = kNB / 4;
+  static_assert(MC == 16 && kNB == 64, "one 16-column chunk, four waves of 16 rows or columns");
+  // a staged tile of op(A) for G, then the four wave partials, then X_l2 and X_l1
+  __shared__ __attribute__((aligned(16))) T Wk[4 * SL > kNB * S ? 4 * SL : kNB * S];
+  __shared__ T Slab[SL];  // B_w - sum
+  __shared__ T Far[kFar ? 4 * NK * 64 : 1];
+  __shared__ int s_ticket, s_abort[3];
+  const int tid = threadIdx.x, lane = tid & 63, fr = lane & 15, fq = lane >> 4;
+  const int wv = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nb = (n + kNB - 1) / kNB, nq = (m + MC - 1) / MC;
-  if (tid == 0) {
-    s_ticket = atomicAdd(ticket, 1);
-    s_abort = 0;
-  }
+  if (tid == 0) s_ticket = atomicAdd(ticket, 1);
+  if (tid < 3) s_abort[tid] = 0;
   __syncthreads();
-  const int tk = s_ticket;
+  const int tk = __builtin_amdgcn_readfirstlane(s_ticket);
   if (tk >= nb * nq) return;
   const int p = tk / nq, q = tk % nq;
   const int w = lower_op ? p : nb - 1 - p;
   const int w0 = w * kNB, bw = min(kNB, n - w0);
   const int c0 = q * MC, mc = min(MC, m - c0);
-  const int r = tid & 63, wv = tid >> 6;
   auto jof = [&](int st) { return lower_op ? st : nb - 1 - st; };
+  auto sidx = [](int k, int c) { return k * MC + (k >> 2) * PAD + c; };
 
-  // the inverse of the diagonal block does not depend on any flag: stage it first
+  // this wave's rows of the inverse, in the order of the products' k
+  T iv[NK];
   {
     const T* D = Dinv + (int64_t)w * kNB * kNB;
 #pragma unroll
-    for (int g = 0; g < 16; ++g) {
-      const int e = tid + 256 * g, i = e / kNB, jj = e % kNB;
-      Dl[(dinv_t ? jj : i) * S + (dinv_t ? i : jj)] = D[e];
+    for (int e = 0; e < NK; ++e) {
+      const int k = 16 * (e / 4) + MF::row(lane, e % 4), r = 16 * wv + fr;
+      iv[e] = D[dinv_t ? k * kNB + r : r * kNB + k];
     }
   }
-  // B_w[r][4 wv .. 4 wv + 3], the entries this thread finishes
+  // B_w, the entries that this lane finishes: rows 16 wv + row(lane, e), column fr
   T bwr[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int c = 4 * wv + e;
-    bwr[e] = (r < bw && c < mc) ? B[(int64_t)(w0 + r) * ldb + c0 + c] : T(0);
+    const int r = 16 * wv + MF::row(lane, e);
+    bwr[e] = (r < bw && fr < mc) ? B[(int64_t)(w0 + r) * ldb + c0 + fr] : T(0);
   }
 
-  // this lane's 16 values of op(A)[w0 + r, j0 + 16 wv + kk] for block j
-  typedef T vec_t __attribute__((ext_vector_type(16 / sizeof(T))));
-  constexpr int VL = 16 / sizeof(T);
-  auto fetch = [&](int st, T* out) {
-    const int j = jof(st), j0 = j * kNB, bj = min(kNB, n - j0), k0 = KW * wv;
-    if (!trans) {
-      const T* row = A + (int64_t)(w0 + min(r, bw - 1)) * lda + j0 + k0;
-      if (VEC && k0 + KW <= bj) {
+  // g = this wave's rows of inv(op(A)_ww) op(A)_wj, j at position st, as the operand of
+  // a product over k in the order of iv (computed transposed, which leaves it so)
+  auto make_g = [&](int st, T (&g)[NK]) __attribute__((always_inline)) {
+    const int j0 = jof(st) * kNB, bj = min(kNB, n - j0);
+    __syncthreads();
+    T v[NK];
 #pragma unroll
-        for (int v = 0; v < KW / VL; ++v) {
-          const vec_t x = *reinterpret_cast<const vec_t*>(row + v * VL);
+    for (int e = 0; e < NK; ++e) {
+      const int i = (tid + 256 * e) / kNB, jj = (tid + 256 * e) % kNB, r = trans ? jj : i, c = trans ? i : jj;
+      const int64_t rr = w0 + min(r, bw - 1);
+      v[e] = c < bj ? A[trans ? (int64_t)(j0 + c) * lda + rr : rr * lda + j0 + c] : T(0);
+    }
 #pragma unroll
-          for (int e = 0; e < VL; ++e) out[v * VL + e] = x[e];
-        }
-      } else {
+    for (int e = 0; e < NK; ++e) {
+      const int i = (tid + 256 * e) / kNB, jj = (tid + 256 * e) % kNB, r = trans ? jj : i, c = trans ? i : jj;
+      Wk[r * S + c] = v[e];
+    }
+    __syncthreads();
 #pragma unroll
-        for (int kk = 0; kk < KW; ++kk) out[kk] = (k0 + kk < bj) ? row[kk] : T(0);
-      }
-    } else {
-      const T* col = A + (int64_t)j0 * lda + w0 + min(r, bw - 1);
+    for (int kt = 0; kt < 4; ++kt) {
+      acc_t t{};
 #pragma unroll
-      for (int kk = 0; kk < KW; ++kk) out[kk] = (k0 + kk < bj) ? col[(int64_t)(k0 + kk) * lda] : T(0);
+      for (int e = 0; e < NK; ++e)
+        t = MF::mma(Wk[(16 * (e / 4) + MF::row(lane, e % 4)) * S + 16 * kt + fr], iv[e], t);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) g[4 * kt + e] = t[e];
     }
   };
-  // X_j rows [0, 64) x chunk columns: 4 values per thread (row e / 16, column e % 16)
-  auto loady = [&](int st, T* out) {
-    const int j0 = jof(st) * kNB, bj = min(kNB, n - j0);
+  T g1[NK], g2[NK];
+  if (p > 0) make_g(p - 1, g1);
+  if (p > 1) make_g(p - 2, g2);
+  T* const far = Far + (kFar ? wv * NK * 64 + lane : 0);
+  if constexpr (kFar) {
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int e = tid + 256 * g, k = e / MC, c = e % MC;
-      out[g] = (k < bj && c < mc) ? B[(int64_t)(j0 + k) * ldb + c0 + c] : T(0);
+    for (int e = 0; e < NK; ++e) far[64 * e] = g2[e];
+  }
+
+  // this lane's values of op(A)[w0 + 16 i + fr, j0 + 16 wv + 4 fq + e], at 4 i + e
+  typedef T vec_t __attribute__((ext_vector_type(16 / sizeof(T))));
+  constexpr int VL = 16 / sizeof(T);
+  auto fetch = [&](int st, T (&out)[NK]) __attribute__((always_inline)) {
+    const int j0 = jof(st) * kNB, bj = min(kNB, n - j0), k0 = 16 * wv + 4 * fq;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int64_t r = w0 + min(16 * i + fr, bw - 1);
+      if (!trans) {
+        const T* row = A + r * lda + j0 + k0;
+        if (VEC && bj == kNB) {
+#pragma unroll
+          for (int v = 0; v < 4 / VL; ++v) {
+            const vec_t x = *reinterpret_cast<const vec_t*>(row + v * VL);
+#pragma unroll
+            for (int e = 0; e < VL; ++e) out[4 * i + v * VL + e] = x[e];
+          }
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) out[4 * i + e] = (k0 + e < bj) ? row[e] : T(0);
+        }
+      } else {
+        const T* col = A + (int64_t)(j0 + k0) * lda + r;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) out[4 * i + e] = (k0 + e < bj) ? col[(int64_t)e * lda] : T(0);
+      }
     }
+  };
+  // rows 16 wv + 4 fq + e of X_j, column fr, from B
+  auto loadx = [&](int st, T (&out)[4]) __attribute__((always_inline)) {
+    const int j0 = jof(st) * kNB, bj = min(kNB, n - j0), k0 = 16 * wv + 4 * fq;
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      out[e] = (k0 + e < bj && fr < mc) ? agent_load(&B[(int64_t)(j0 + k0 + e) * ldb + c0 + fr]) : T(0);
+  };
+  // one more poll of a wait: false once it gives up
+  auto go_on = [&](int64_t& it, int stage) -> bool {
+    if (spin_limit >= 0 && ++it <= spin_limit &&
+        ((it & 7) != 0 || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0))
+      return true;
+    if (lane == 0) {
+      atomicExch(err, 1);
+      s_abort[stage] = 1;
+    }
+    return false;
   };
   // wait until block st's flag is raised, then take every later flag already
   // raised (up to the window); false when the wait gave up
   int ready = 0;
   auto wait_for = [&](int st) -> bool {
-    if (tid == 0) {
-      int64_t it = 0;
-      const int32_t* f = &flags[jof(st) * nq + q];
-      if (spin_limit < 0) {
-        atomicExch(err, 1);
-        s_abort = 1;
-      }
-      while (!s_abort && __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch) {
-        if (++it > spin_limit || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-          atomicExch(err, 1);
-          s_abort = 1;
-          break;
-        }
-        __builtin_amdgcn_s_sleep(1);
-      }
-      int t2 = st + 1;
-      while (t2 < p && t2 < st + kFlagWindow &&
-             __hip_atomic_load(&flags[jof(t2) * nq + q], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == epoch)
-        ++t2;
-      s_ready = t2;
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    const int32_t* f = &flags[jof(st) * nq + q];
+    int64_t it = 0;
+    bool go = spin_limit >= 0 || go_on(it, 0);
+    while (go && __hip_atomic_load(f, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != epoch) {
+      go = go_on(it, 0);
+      __builtin_amdgcn_s_sleep(1);
     }
-    __syncthreads();
-    if (s_abort) return false;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");
-    ready = s_ready;
+    if (!go) return false;
+    const int t2 = st + 1 + lane;
+    const bool up = lane < kFlagWindow - 1 && t2 < p &&
+                    __hip_atomic_load(&flags[jof(min(t2, p - 1)) * nq + q], __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT) == epoch;
+    const uint64_t down = ~(uint64_t)__ballot(up);  // (lane 63 is never up)
+    ready = __builtin_amdgcn_readfirstlane(st + 1 + __builtin_ctzll(down));
+    asm volatile("" ::: "memory");
     return true;
   };
-
-  // Gs[i][r][16 wv + kk] = sum_k inv(op(A)_ww)[r][k] op(A)_w,l[k][16 wv + kk], l at position st
-  auto make_g = [&](int st, T* gs) {
-    T t[KW];
-    fetch(st, t);
+  // words o[e] of block st from the ring, once all of them carry its tag
+  uint64_t* const ring = mail + (int64_t)q * kMailRing * kMailSlot;
+  auto take = [&](int st, int o0, int step, T (&out)[4], int stage) -> bool {
+    const uint64_t* box = ring + (st % kMailRing) * kMailSlot + o0;
+    const uint32_t tag = (uint32_t)epoch + (uint32_t)(st / kMailRing);
+    int64_t it = 0;
+    if (spin_limit < 0 && !go_on(it, stage)) return false;
+    for (;;) {
+      uint64_t lo[4], hi[4];
+      bool got = true;
 #pragma unroll
-    for (int kk = 0; kk < KW; ++kk) Wk[r * S + KW * wv + kk] = t[kk];
-    __syncthreads();
-    T g[KW];
+      for (int e = 0; e < 4; ++e) {
+        lo[e] = agent_load(box + step * e);
+        if constexpr (sizeof(T) == 8) hi[e] = agent_load(box + step * e + kNB * MC);
+      }
 #pragma unroll
-    for (int kk = 0; kk < KW; ++kk) g[kk] = T(0);
-#pragma unroll 4
-    for (int k = 0; k < kNB; ++k) {
-      const T d = Dl[r * S + k];
-#pragma unroll
-      for (int kk = 0; kk < KW; ++kk) g[kk] += d * Wk[k * S + KW * wv + kk];
+      for (int e = 0; e < 4; ++e) {
+        got = got && (uint32_t)(lo[e] >> 32) == tag;
+        if constexpr (sizeof(T) == 8) {
+          got = got && (uint32_t)(hi[e] >> 32) == tag;
+          out[e] = __builtin_bit_cast(double, (hi[e] << 32) | (uint32_t)lo[e]);
+        } else {
+          out[e] = __builtin_bit_cast(float, (uint32_t)lo[e]);
+        }
+      }
+      if (__ballot(!got) == 0) return true;
+      if (!go_on(it, stage)) return false;
     }
-#pragma unroll
-    for (int kk = 0; kk < KW; ++kk) gs[r * S + KW * wv + kk] = g[kk];
-    __syncthreads();
   };
-  const int l1 = p - 1, l2 = p - 2;  // positions of the last two dependencies
-  if (p > 0) make_g(l1, Gs[0]);
-  if (p > 1) make_g(l2, Gs[1]);
 
   // the walk over the blocks before l2
   const int nwalk = max(p - 2, 0);
-  T acc[MC];
+  acc_t acc[4];
 #pragma unroll
-  for (int c = 0; c < MC; ++c) acc[c] = T(0);
+  for (int i = 0; i < 4; ++i) acc[i] = acc_t{};
   {
-    T a_cur[KW], a_nxt[KW], y_cur[4], y_nxt[4];
-    bool y_pre = false;
+    T a_cur[NK], a_nxt[NK], x_cur[4], x_nxt[4];
+    bool x_pre = false;
     if (nwalk > 0) fetch(0, a_cur);
     for (int st = 0; st < nwalk; ++st) {
-      if (st >= ready) {
-        if (!wait_for(st)) return;
-        y_pre = false;
-      }
-      if (y_pre) {
+      if (x_pre) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) y_cur[e] = y_nxt[e];
+        for (int e = 0; e < 4; ++e) x_cur[e] = x_nxt[e];
+      } else if (st >= ready && st >= p - kMailReach) {
+        if (!take(st, (16 * wv + 4 * fq) * MC + fr, MC, x_cur, 0)) break;
       } else {
-        loady(st, y_cur);
+        if (st >= ready && !wait_for(st)) break;
+        loadx(st, x_cur);
       }
-      T* ys = Wk + (st & 1) * SL;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) ys[tid + 256 * e] = y_cur[e];
-      __syncthreads();
       if (st + 1 < nwalk) fetch(st + 1, a_nxt);
-      y_pre = st + 1 < nwalk && st + 1 < ready;
-      if (y_pre) loady(st + 1, y_nxt);
-      const T* yk = ys + KW * wv * MC;
+      x_pre = st + 1 < nwalk && st + 1 < ready;
+      if (x_pre) loadx(st + 1, x_nxt);
 #pragma unroll
-      for (int kk = 0; kk < KW; ++kk) {
-        const T a = a_cur[kk];
+      for (int e = 0; e < 4; ++e)
 #pragma unroll
-        for (int c = 0; c < MC; ++c) acc[c] += a * yk[kk * MC + c];
-      }
+        for (int i = 0; i < 4; ++i) acc[i] = MF::mma(a_cur[4 * i + e], x_cur[e], acc[i]);
 #pragma unroll
-      for (int kk = 0; kk < KW; ++kk) a_cur[kk] = a_nxt[kk];
+      for (int e = 0; e < NK; ++e) a_cur[e] = a_nxt[e];
     }
   }
 
-  // Z = inv(op(A)_ww) (B_w - sum): reduce the wave partials into Slab, then
-  // lane r, columns 4 wv .. 4 wv + 3
-  __syncthreads();
+  // Z = inv(op(A)_ww) (B_w - sum): the wave partials reduced, then 16 rows a wave
+  __syncthreads();  // every wave is done with the staged tile
 #pragma unroll
-  for (int c = 0; c < MC; ++c) Part[wv * SL + r * MC + c] = acc[c];
+  for (int i = 0; i < 4; ++i)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) Wk[wv * SL + sidx(16 * i + MF::row(lane, e), fr)] = acc[i][e];
   __syncthreads();
+  if (s_abort[0]) return;
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    const int c = 4 * wv + e, o = r * MC + c;
-    const T sum = Part[o] + Part[SL + o] + Part[2 * SL + o] + Part[3 * SL + o];
-    Slab[o] = (r < bw && c < mc) ? bwr[e] - sum : T(0);
+    const int r = 16 * wv + MF::row(lane, e), o = sidx(r, fr);
+    const T sum = Wk[o] + Wk[SL + o] + Wk[2 * SL + o] + Wk[3 * SL + o];
+    Slab[o] = (r < bw && fr < mc) ? bwr[e] - sum : T(0);
   }
   __syncthreads();
-  T x[4] = {T(0), T(0), T(0), T(0)};
-#pragma unroll 8
-  for (int k = 0; k < kNB; ++k) {
-    const T d = Dl[r * S + k];
+  // f x slab, in f32 as four sums of 16 terms (less rounding than one of 64)
+  auto product = [&](const T (&f)[NK], const T* slab) __attribute__((always_inline)) -> acc_t {
+    constexpr int NP = sizeof(T) == 4 ? 4 : 1;
+    acc_t t[NP];
 #pragma unroll
-    for (int e = 0; e < 4; ++e) x[e] += d * Slab[k * MC + 4 * wv + e];
-  }
-
-  // x -= G X_l for the dependency at position st, once its flag is raised
-  auto apply_g = [&](int st, const T* gs) -> bool {
-    if (st >= ready && !wait_for(st)) return false;
+    for (int i = 0; i < NP; ++i) t[i] = acc_t{};
+#pragma unroll
+    for (int e = 0; e < NK; ++e)
+      t[e % NP] = MF::mma(f[e], slab[sidx(16 * (e / 4) + MF::row(lane, e % 4), fr)], t[e % NP]);
+    if constexpr (NP == 4) return (t[0] + t[1]) + (t[2] + t[3]);
+    return t[0];
+  };
+  acc_t x = product(iv, Slab);
+  // x -= G X for the dependency at position st, 16 of whose rows each wave takes
+  auto apply_g = [&](int st, const T (&g)[NK], int stage) __attribute__((always_inline)) -> bool {
     T y[4];
-    loady(st, y);
-    __syncthreads();  // every wave is done reading Slab and Part
+    T* const slab = Wk + (stage - 1) * SL;
+    if (take(st, 16 * MC * wv + lane, 4 * MC, y, stage)) {
 #pragma unroll
-    for (int e = 0; e < 4; ++e) Slab[tid + 256 * e] = y[e];
-    __syncthreads();
-    T gy[MC];
-#pragma unroll
-    for (int c = 0; c < MC; ++c) gy[c] = T(0);
-    const T* yk = Slab + KW * wv * MC;
-#pragma unroll
-    for (int kk = 0; kk < KW; ++kk) {
-      const T gv = gs[r * S + KW * wv + kk];
-#pragma unroll
-      for (int c = 0; c < MC; ++c) gy[c] += gv * yk[kk * MC + c];
+      for (int e = 0; e < 4; ++e) slab[sidx(16 * wv + 4 * e + fq, fr)] = y[e];
     }
-#pragma unroll
-    for (int c = 0; c < MC; ++c) Part[wv * SL + r * MC + c] = gy[c];
     __syncthreads();
+    if (s_abort[stage]) return false;
+    const acc_t t = product(g, slab);
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      const int o = r * MC + 4 * wv + e;
-      x[e] -= Part[o] + Part[SL + o] + Part[2 * SL + o] + Part[3 * SL + o];
-    }
+    for (int e = 0; e < 4; ++e) x[e] -= t[e];
     return true;
   };
-  if (p > 1 && !apply_g(l2, Gs[1])) return;
-  if (p > 0 && !apply_g(l1, Gs[0])) return;
+  if (p > 1) {
+    if constexpr (kFar) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e)
-    if (r < bw && 4 * wv + e < mc) B[(int64_t)(w0 + r) * ldb + c0 + 4 * wv + e] = x[e];
-  // Each wave releases its own stores at agent scope (a release fence: the
-  // seq_cst __threadfence would also invalidate the L2 after every block);
-  // thread 0's release store of the flag follows the barrier.
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      for (int e = 0; e < NK; ++e) g2[e] = far[64 * e];
+    }
+    if (!apply_g(p - 2, g2, 1)) return;
+  }
+  if (p > 0 && !apply_g(p - 1, g1, 2)) return;
+  if (p + 1 < nb) {
+    uint64_t* box = ring + (p % kMailRing) * kMailSlot;
+    const uint64_t tag = (uint64_t)((uint32_t)epoch + (uint32_t)(p / kMailRing)) << 32;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int r = 16 * wv + MF::row(lane, e);
+      const T v = r < bw ? x[e] : T(0);
+      if constexpr (sizeof(T) == 8) {
+        const uint64_t u = __builtin_bit_cast(uint64_t, v);
+        agent_store(box + r * MC + fr, tag | (uint32_t)u);
+        agent_store(box + kNB * MC + r * MC + fr, tag | (u >> 32));
+      } else {
+        agent_store(box + r * MC + fr, tag | __builtin_bit_cast(uint32_t, v));
+      }
+    }
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+    const int r = 16 * wv + MF::row(lane, e);
+    if (r < bw && fr < mc) agent_store(&B[(int64_t)(w0 + r) * ldb + c0 + fr], (T)x[e]);
+  }
+  if (p + kMailReach + 1 >= nb) return;  // no position reads this flag
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores have reached memory
   __syncthreads();
-  if (tid == 0) __hip_atomic_store(&flags[w * nq + q], epoch, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid == 0) __hip_atomic_store(&flags[w * nq + q], epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 }  // namespace
@@ -478,8 +562,8 @@ hipError_t launch_trtri_blocks(int n, const TS* A, int64_t lda, bool trans, bool
 template <typename T>
 hipError_t launch_trsm_persistent(int n, int m, const T* A, int64_t lda, bool trans, bool lower_op,
                                   const T* Dinv, bool dinv_t, T* B, int64_t ldb, int32_t* ticket,
-                                  int32_t* flags, int32_t epoch, int32_t* err, int64_t spin_limit,
-                                  const int32_t* gate, hipStream_t s) {
+                                  int32_t* flags, uint64_t* mail, int32_t epoch, int32_t* err,
+                                  int64_t spin_limit, const int32_t* gate, hipStream_t s) {
   if (n <= 0 || m <= 0) return hipSuccess;
   const int nb = (n + kNB - 1) / kNB, nq = (m + kSolveChunk - 1) / kSolveChunk;
   hipError_t e = launch_fill_i32(ticket, 0, 1, s);
@@ -487,10 +571,10 @@ hipError_t launch_trsm_persistent(int n, int m, const T* A, int64_t lda, bool tr
   const bool vec = (reinterpret_cast<uintptr_t>(A) % 16 == 0) && ((lda * sizeof(T)) % 16 == 0);
   if (vec)
     hipLaunchKernelGGL((trsm_persistent_kernel<T, true>), dim3(nb * nq), dim3(256), 0, s, n, m, A, lda, trans,
-                       lower_op, Dinv, dinv_t, B, ldb, ticket, flags, epoch, err, spin_limit, gate);
+                       lower_op, Dinv, dinv_t, B, ldb, ticket, flags, mail, epoch, err, spin_limit, gate);
   else
     hipLaunchKernelGGL((trsm_persistent_kernel<T, false>), dim3(nb * nq), dim3(256), 0, s, n, m, A, lda, trans,
-                       lower_op, Dinv, dinv_t, B, ldb, ticket, flags, epoch, err, spin_limit, gate);
+                       lower_op, Dinv, dinv_t, B, ldb, ticket, flags, mail, epoch, err, spin_limit, gate);
   return hipGetLastError();
 }
 
@@ -501,11 +585,11 @@ template hipError_t launch_trtri_blocks<float, float>(int, const float*, int64_t
 template hipError_t launch_trtri_blocks<float, double>(int, const float*, int64_t, bool, bool, float*,
                                                        const int32_t*, hipStream_t, int32_t*);
 template hipError_t launch_trsm_persistent<double>(int, int, const double*, int64_t, bool, bool, const double*,
-                                                   bool, double*, int64_t, int32_t*, int32_t*, int32_t, int32_t*,
-                                                   int64_t, const int32_t*, hipStream_t);
+                                                   bool, double*, int64_t, int32_t*, int32_t*, uint64_t*, int32_t,
+                                                   int32_t*, int64_t, const int32_t*, hipStream_t);
 template hipError_t launch_trsm_persistent<float>(int, int, const float*, int64_t, bool, bool, const float*, bool,
-                                                  float*, int64_t, int32_t*, int32_t*, int32_t, int32_t*, int64_t,
-                                                  const int32_t*, hipStream_t);
+                                                  float*, int64_t, int32_t*, int32_t*, uint64_t*, int32_t, int32_t*,
+                                                  int64_t, const int32_t*, hipStream_t);
 template hipError_t launch_trsm_rows<double>(int, int, double*, int64_t, const double*, int64_t,
                                              const int32_t*, hipStream_t);
 template hipError_t launch_trsm_rows<float>(int, int, float*, int64_t, const float*, int64_t, const int32_t*,

@@ -51,20 +51,31 @@ constexpr int kStepRows = 8192;
 // the bound on its flag waits (2^22 polls: well over 0.1 s, far above any real wait).
 constexpr int kSolveChunkHost = 16;
 constexpr int64_t kSpinLimit = 1ll << 22;
+// The blocks that the solve's workgroups hand to their successors: a ring of kMailRing
+// blocks of kMailSlot 64-bit words (a 32-bit half and its tag) per column chunk, for
+// up to kMailChunks chunks a launch (16 MB).
+constexpr int kMailRing = 8;
+constexpr int kMailSlot = 2 * kNB * kSolveChunkHost;
+constexpr int kMailChunks = 128;
+inline int64_t solve_chunks(int64_t m) { return (m + kSolveChunkHost - 1) / kSolveChunkHost; }
+inline int64_t solve_mail_words(int64_t chunks) { return chunks * kMailRing * kMailSlot; }
+// Tags that a launch of n rows takes: one per lap of the ring.
+inline int solve_epochs(int n) { return ((n + kNB - 1) / kNB + kMailRing - 1) / kMailRing; }
 
 // Rows that one launch of the triangular solve takes for m right-hand sides
 // (trsm_split): all of them up to 64 columns, where the chain of 64-row hops
-// bounds it; with more columns about as many as keep its products, which run on
-// the VALU, shorter than that chain -- n * m = 1.5M (f64), 3M (f32), the rest as
-// MFMA products between launches.  Measured (us) at 1024 / 2048 / 4096 rows / all:
-// f64 n = 4096 m = 300 1390 / 1063 / 873 / 869, m = 1500 2523 / 2749 / 3607 / 3606;
-// f64 n = 12000 m = 100 5304 / 4274 / 3416 / 2300, m = 500 6202 / 5162 / 4951 / 8342;
-// f32 n = 12000 m = 1500 8009 / 7292 / 7094 / 9491.
+// bounds it; with more columns n * m = 6M, about as many as keep its products
+// shorter than that chain, the rest as products with larger tiles between launches.
+// Measured (us, L / L^T) at 1.5M / 3M / 6M / 12M: f64 n = 4096 m = 1500 1494, 1460 / 1192,
+// 1185 / 1069, 1116 / -, n = 12000 m = 500 3707, 3663 / 2909, 3110 / 2562, 3091 / -; f32
+// n = 4096 m = 1500 942, 1001 / 804, 827 / 705, 757 / 707, 840, n = 12000 m = 500
+// 2325, 2451 / 1900, 2047 / 1654, 1924 / 1709, 2312; m = 1500 4698 / 4258 / 4081 / 3977,
+// 4746 / 4301 / 4338 / 4721.
 constexpr int kSolveMaxCols = 32768;
 template <typename T>
 inline int solve_split(int m) {
   if (m <= 64) return INT32_MAX;
-  const int rows = (sizeof(T) == 8 ? 1500000 : 3000000) / m / kNB * kNB;
+  const int rows = 6000000 / m / kNB * kNB;
   return rows > kNB ? rows : kNB;
 }
 // Flags that the largest of those launches needs for order n.

@@ -28,6 +28,7 @@ struct llh_context {
   Buffer mixed_scale; // its diagonal scaling (f16 factor)
   Buffer half_panel;  // f16 copy of the panel of the f16 factor's trailing SYRK
   Buffer sync;        // ticket / error / flags of the one-launch solve
+  Buffer mail;        // its blocks in flight
   Buffer fwd_y;       // right-hand sides of the forward substitution fused into the factor
   Buffer host_stage[2];  // page-locked host staging of the plain forms (hipHostMalloc)
   int32_t epoch = 1;

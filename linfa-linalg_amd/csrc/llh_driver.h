@@ -7,15 +7,18 @@
 namespace llh {
 
 // Device words of the one-launch triangular solve: ticket counter, error word
-// and one flag per (64-row block, 16-column chunk).  *epoch is the owner's
-// counter (a context's or a server stream's): the next value the flags have
-// never held; each launch takes it and advances it at once, so no later launch
-// can reuse an epoch whatever path the caller takes afterwards.  The error word
+// and one flag per (64-row block, 16-column chunk), and the rings of blocks in
+// flight (kMailRing), both zeroed when allocated.  *epoch is the owner's
+// counter (a context's or a server stream's): the next value that neither has
+// ever held; each launch takes solve_epochs(n) of them and advances it at once, so
+// no later launch can reuse one whatever path the caller takes afterwards.  The error word
 // is cleared once per call (solve_sync_begin), not per sweep, so a sweep that
 // gave up stays visible after the sweeps that follow it.
 struct SolveSync {
   int32_t* words = nullptr;  // [0] ticket, [1] error, [2..] flags
   int64_t nflags = 0;
+  uint64_t* mail = nullptr;
+  int64_t nmail = 0;  // 16-column chunks that mail has room for
   int32_t* epoch = nullptr;
   int64_t spin_limit = kSpinLimit;  // bound on each flag wait (negative: give up at once)
   // Device word of solves of more than 64 columns with inverses of their own

@@ -221,14 +221,15 @@ hipError_t launch_trtri_blocks(int n, const TS* A, int64_t lda, bool trans, bool
                                const int32_t* gate, hipStream_t s, int32_t* wild = nullptr);
 // k_trsm.hip: one-launch blocked solve op(A) X = B (B row-major n x m) using the
 // diagonal-block inverses Dinv (transposed when dinv_t).  ticket/flags/err are
-// device words (flags: one per 64-row block and 16-column chunk), epoch a value
-// the flags have never held.  *err becomes non-zero if a wait exceeded spin_limit
+// device words (flags: one per 64-row block and 16-column chunk), mail holds
+// solve_mail_words(1) zeroed words per 16-column chunk, and epoch .. epoch +
+// solve_epochs(n) - 1 are values that neither has ever held.  *err becomes non-zero if a wait exceeded spin_limit
 // (a negative spin_limit: at the first wait).
 template <typename T>
 hipError_t launch_trsm_persistent(int n, int m, const T* A, int64_t lda, bool trans, bool lower_op,
                                   const T* Dinv, bool dinv_t, T* B, int64_t ldb, int32_t* ticket,
-                                  int32_t* flags, int32_t epoch, int32_t* err, int64_t spin_limit,
-                                  const int32_t* gate, hipStream_t s);
+                                  int32_t* flags, uint64_t* mail, int32_t epoch, int32_t* err,
+                                  int64_t spin_limit, const int32_t* gate, hipStream_t s);
 
 // k_mixed.hip: conversions, symmetric residual and norms of the refinement.
 // Y = diag(rs) X diag(cs) in f32 (null scales are 1).

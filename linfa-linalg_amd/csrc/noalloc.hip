@@ -2,7 +2,7 @@
 // and solves as llh_dev_solvec_d, with the scratch those take from the
 // context's grow-only buffers (the inverses of the 64 x 64 diagonal blocks, the
 // right-hand sides of the forward substitution fused into the factor, and the
-// ticket, error word and flags of the one-launch solve) placed in a static
+// ticket, error word, flags and rings of the one-launch solve) placed in a static
 // device array instead.  Each GPU the library runs on holds its own copy of the
 // array until the process ends; llh_context_create locates it once per device
 // (hipGetSymbolAddress with that device current) and every later use goes
@@ -17,10 +17,12 @@
 
 namespace {
 
-constexpr size_t kSyncBytes = 16u * 1024u;          // [0] ticket, [1] error word, [2..] flags
+constexpr size_t kSyncBytes = 32u * 1024u;          // [0] ticket, [1] error word, [2..] flags
 constexpr size_t kInvBytes = 8u * 1024u * 1024u;    // inverses of the diagonal blocks
 constexpr size_t kFwdBytes = 8u * 1024u * 1024u;    // fused forward substitution: n x m, m <= 64
-constexpr size_t kScratchBytes = kSyncBytes + kInvBytes + kFwdBytes;
+constexpr size_t kMailChunksNoalloc = 4;            // 64 columns a launch of the one-launch solve
+constexpr size_t kMailBytes = kMailChunksNoalloc * llh::kMailRing * llh::kMailSlot * sizeof(uint64_t);
+constexpr size_t kScratchBytes = kSyncBytes + kMailBytes + kInvBytes + kFwdBytes;
 static_assert(kScratchBytes == LLH_NOALLOC_SCRATCH_BYTES, "the header states the array's size");
 static_assert(kInvBytes / (llh::kNB * sizeof(double)) == LLH_NOALLOC_MAX_N, "the header states the bound");
 static_assert(kFwdBytes == (size_t)LLH_NOALLOC_MAX_N * 64 * sizeof(double),
@@ -47,7 +49,7 @@ DeviceScratch g_scratch[kMaxDevices];
 
 namespace llh {
 
-// Locates this device's copy of the array and clears its flags (they start at
+// Locates this device's copy of the array and clears its flags and rings (they start at
 // 0, below every epoch handed out).  Runs with `device` current, once per
 // device; later calls return the first outcome.
 hipError_t noalloc_init(int device, hipStream_t s) {
@@ -59,7 +61,8 @@ hipError_t noalloc_init(int device, hipStream_t s) {
   void* p = nullptr;
   hipError_t e = hipGetSymbolAddress(&p, HIP_SYMBOL(scratch));
   if (e == hipSuccess && p == nullptr) e = hipErrorInvalidSymbol;
-  if (e == hipSuccess) e = launch_fill_i32(static_cast<int32_t*>(p), 0, (int64_t)(kSyncBytes / 4), s);
+  if (e == hipSuccess) e = launch_fill_i32(static_cast<int32_t*>(p), 0,
+                                           (int64_t)((kSyncBytes + kMailBytes) / 4), s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) (void)hipGetLastError();
   d.status = e;
@@ -93,11 +96,13 @@ extern "C" llh_status llh_dev_solvec_noalloc_d(llh_context* ctx, size_t n, doubl
     epoch = &d.epoch;
   }
   hipStream_t s = ctx->stream;
-  double* dinv = reinterpret_cast<double*>(base + kSyncBytes);
-  double* fwd_y = reinterpret_cast<double*>(base + kSyncBytes + kInvBytes);
+  double* dinv = reinterpret_cast<double*>(base + kSyncBytes + kMailBytes);
+  double* fwd_y = reinterpret_cast<double*>(base + kSyncBytes + kMailBytes + kInvBytes);
   SolveSync sync;
   sync.words = reinterpret_cast<int32_t*>(base);
   sync.nflags = (int64_t)(kSyncBytes / 4) - 2;
+  sync.mail = reinterpret_cast<uint64_t*>(base + kSyncBytes);
+  sync.nmail = kMailChunksNoalloc;
   sync.epoch = epoch;
   sync.spin_limit = ctx->spin_limit;
   // the lookahead streams exist from llh_context_create on; nothing is created here

@@ -114,6 +114,7 @@ struct StreamState {
   SolveSync sync;
   int32_t epoch = 1;  // the flags' epoch counter of this stream's solves
   void* sync_buf = nullptr;
+  void* mail_buf = nullptr;
   size_t sync_bytes = 0;
 };
 
@@ -217,6 +218,20 @@ hipError_t ensure_sync(llh_server* s, StreamState& st, int n, int m) {
   const size_t want = (2 + nb * nq) * sizeof(int32_t);
   st.sync.epoch = &st.epoch;
   st.sync.spin_limit = s->spin_limit.load();
+  const int64_t chunks = std::min<int64_t>(std::max<size_t>(nq, 1), kMailChunks);
+  if (st.sync.nmail < chunks) {
+    hipError_t e = hipStreamSynchronize(st.s);
+    if (e != hipSuccess) return e;
+    if (st.mail_buf) (void)hipFree(st.mail_buf);
+    st.mail_buf = nullptr;
+    st.sync.mail = nullptr;
+    st.sync.nmail = 0;
+    const int64_t words = solve_mail_words(chunks);
+    if ((e = hipMalloc(&st.mail_buf, (size_t)words * 8)) != hipSuccess) return e;
+    if ((e = launch_fill_i32(static_cast<int32_t*>(st.mail_buf), 0, 2 * words, st.s)) != hipSuccess) return e;
+    st.sync.mail = static_cast<uint64_t*>(st.mail_buf);
+    st.sync.nmail = chunks;
+  }
   if (st.sync_bytes >= want) return hipSuccess;
   hipError_t e = hipStreamSynchronize(st.s);
   if (e != hipSuccess) return e;
@@ -229,7 +244,6 @@ hipError_t ensure_sync(llh_server* s, StreamState& st, int n, int m) {
     return e;
   st.sync.words = static_cast<int32_t*>(st.sync_buf);
   st.sync.nflags = (int64_t)(bytes / 4) - 2;
-  st.epoch = 1;
   return hipSuccess;
 }
 
@@ -819,6 +833,7 @@ void llh_server_destroy(llh_server* s) {
   for (auto& st : s->streams) {
     if (st.s) (void)hipStreamSynchronize(st.s);
     if (st.sync_buf) (void)hipFree(st.sync_buf);
+    if (st.mail_buf) (void)hipFree(st.mail_buf);
     if (st.s) (void)hipStreamDestroy(st.s);
   }
   for (auto e : s->event_pool) (void)hipEventDestroy(e);
