@@ -144,12 +144,12 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, 2) void panel_step_kernel(TS* a, 
   }
 
   // L(k, k-1)'s strip c times this wave's strip (!left) or the transposed rows (left),
-  // added to x.  In f32 it is summed by itself first: added term by term, every
-  // partial sum would be rounded at the size of x.
+  // added to x, summed by itself first: added term by term, every partial sum would
+  // be rounded at the size of x (n = 512, f64: error of L 2.6e-16 against 1.8e-16).
   auto apply = [&](typename MS::acc_t& x, int c, auto left) __attribute__((always_inline)) {
     typename MS::acc_t t;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) t[r] = sizeof(TS) == 8 ? x[r] : TS(0);
+    for (int r = 0; r < 4; ++r) t[r] = TS(0);
 #pragma unroll
     for (int s = 0; s < W; ++s) {
       const TS v = sm.c.lk[(W * c + fr) * LK + W * fq + s];
@@ -159,7 +159,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, 2) void panel_step_kernel(TS* a, 
         t = MS::mma(sm.c.lk[(W * g + fr) * LK + W * fq + s], v, t);
     }
 #pragma unroll
-    for (int r = 0; r < 4; ++r) x[r] = sizeof(TS) == 8 ? t[r] : x[r] + t[r];
+    for (int r = 0; r < 4; ++r) x[r] += t[r];
   };
   using Left = std::true_type;
   using Diag = std::false_type;
