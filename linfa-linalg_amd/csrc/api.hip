@@ -275,8 +275,8 @@ llh_status factor_plain(llh_context* ctx, size_t n, T* a, ptrdiff_t rs, ptrdiff_
   void* dv = nullptr;
   CHECK_HIP(ctx_buffer(ctx, 0, n * n * sizeof(T), &dv), "device buffer");
   T* d = static_cast<T*>(dv);
-  void* dinv = nullptr;
-  CHECK_HIP(ctx_dinv(ctx, (int)n, sizeof(T), &dinv), "inverse buffer");
+  void* dinv = nullptr;  // (the small factor makes inverses for solves only)
+  if ((int)n > small_max<T>()) CHECK_HIP(ctx_dinv(ctx, (int)n, sizeof(T), &dinv), "inverse buffer");
   CHECK_HIP(hipMemcpyAsync(d, h, n * n * sizeof(T), hipMemcpyHostToDevice, ctx->stream), "upload");
   CHECK_HIP(potrf_enqueue<T>(d, (int64_t)n, (int)n, ctx->d_info, clean, static_cast<T*>(dinv), ctx->stream, nullptr,
                             false, ctx_lookahead(ctx)),
@@ -581,8 +581,8 @@ llh_status dev_potrf(llh_context* ctx, size_t n, T* a, size_t lda, int zero_uppe
   if (n == 0) return ok(err);
   if (a == nullptr || lda < n) return invalid(err, "null matrix or lda < n");
   if (n > 0x7fffffff) return invalid(err, "matrix too large");
-  void* dinv = nullptr;
-  CHECK_HIP(ctx_dinv(ctx, (int)n, sizeof(T), &dinv), "inverse buffer");
+  void* dinv = nullptr;  // (the small factor makes inverses for solves only)
+  if ((int)n > small_max<T>()) CHECK_HIP(ctx_dinv(ctx, (int)n, sizeof(T), &dinv), "inverse buffer");
   CHECK_HIP(potrf_enqueue<T>(a, (int64_t)lda, (int)n, ctx->d_info, zero_upper != 0, static_cast<T*>(dinv),
                             ctx->stream, ctx->profiler(), false, ctx_lookahead(ctx)),
             "potrf");
