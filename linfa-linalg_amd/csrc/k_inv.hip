@@ -6,7 +6,8 @@
 // What bounds it: MFMA and, for small orders, the longest sum of one 64 x 64 tile
 // (n products of 16 x 16 x 4 on four SIMDs); 64 x 64 tiles keep that short and the
 // chip full.  Against the recursion with one product per launch and full
-// operands, n = 3000 f64: 7.1 -> 1.8 ms with the factor (n = 8192 36.0 -> 15.7).
+// operands, n = 3000 f64: 7.1 -> 1.8 ms with the factor (n = 8192 36.0 -> 15.7); with
+// the tiles' order and addresses below 1.58.
 #include "k_gemm_impl.h"
 #include "llh_common.h"
 #include "llh_kernels.h"
@@ -21,8 +22,7 @@ constexpr int kInvRun = 128;
 // acc = sum over k in [klo, khi) of op(A)[m0 + i, k] B[k, n0 + j] for this wave's
 // part of a 64 x 64 tile; A is M x K row-major (TA: K x M), B is K x N row-major.
 // Slabs of kInvK go through LDS in k-major order, the next one loaded into
-// registers while the current one is multiplied.  Rows and columns beyond M, N
-// and k beyond khi read as zero.  The sum is taken in runs of kInvRun k, each
+// registers while the current one is multiplied.  k beyond khi reads as zero.  The sum is taken in runs of kInvRun k, each
 // added to the total as a whole: summed straight through, the rounding grows with
 // the order (f32 inverse, n = 3000: 1.2e-6 against 4.3e-7 relative).
 template <typename T, bool TA>
@@ -35,22 +35,35 @@ __device__ __forceinline__ void inv_tile(int M, int N, int klo, int khi, const T
   const int t = threadIdx.x, lane = t & 63, wave = t >> 6, fr = lane & 15, fk = lane >> 4;
   const int wm = (wave >> 2) * 32, wn = (wave & 3) * 16;
   T va[PER], vb[PER];
+  // This thread's pieces: addresses of slab klo, advanced slab by slab (computed
+  // anew for each they cost the last level's first product 131 us instead of 116, W^T W
+  // 242 instead of 223).  Rows and columns
+  // beyond M, N repeat the last one; what they give is not stored.
+  const T *pa[PER], *pb[PER];
+  int ka[PER], kb[PER];
+#pragma unroll
+  for (int p = 0; p < PER; ++p) {
+    const int e = t + p * kInvT;
+    ka[p] = TA ? e / 64 : e % kInvK;
+    kb[p] = e / 64;
+    const int64_t gr = min(m0 + (TA ? e % 64 : e / kInvK), M - 1), gk = klo + ka[p];
+    pa[p] = TA ? A + gk * lda + gr : A + gr * lda + gk;
+    pb[p] = B + (int64_t)(klo + kb[p]) * ldb + min(n0 + e % 64, N - 1);
+  }
+  const int64_t da = TA ? kInvK * lda : kInvK, db = kInvK * ldb;
   auto load = [&](int k0) __attribute__((always_inline)) {
+    const bool whole = k0 + kInvK <= khi;
 #pragma unroll
     for (int p = 0; p < PER; ++p) {
-      const int e = t + p * kInvT;
-      const int r = TA ? e % 64 : e / kInvK, k = TA ? e / 64 : e % kInvK;
-      const bool in = m0 + r < M && k0 + k < khi;
-      const int64_t gr = min(m0 + r, M - 1), gk = min(k0 + k, khi - 1);
-      const T x = TA ? A[gk * lda + gr] : A[gr * lda + gk];
-      va[p] = in ? x : T(0);
-    }
-#pragma unroll
-    for (int p = 0; p < PER; ++p) {
-      const int e = t + p * kInvT, c = e % 64, k = e / 64;
-      const bool in = n0 + c < N && k0 + k < khi;
-      const T x = B[(int64_t)min(k0 + k, khi - 1) * ldb + min(n0 + c, N - 1)];
-      vb[p] = in ? x : T(0);
+      if (whole) {
+        va[p] = *pa[p];
+        vb[p] = *pb[p];
+      } else {
+        va[p] = k0 + ka[p] < khi ? *pa[p] : T(0);
+        vb[p] = k0 + kb[p] < khi ? *pb[p] : T(0);
+      }
+      pa[p] += da;
+      pb[p] += db;
     }
   };
   auto store = [&](int buf) __attribute__((always_inline)) {
@@ -102,8 +115,15 @@ template <typename T, bool FIRST>
 __global__ __launch_bounds__(kInvT) void inv_level_kernel(int n, int h, const T* __restrict__ L, int64_t lda, T* W,
                                                           int64_t ldw, T* tmp) {
   const int o = 2 * h * blockIdx.y, n2 = min(h, n - o - h), nt = h / 64;
-  const int m0 = (blockIdx.x / nt) * 64, n0 = (blockIdx.x % nt) * 64;
-  if (m0 >= n2) return;
+  const int mt = (n2 + 63) / 64, tiles = mt * nt, half = (tiles + 1) / 2;
+  int t0 = blockIdx.x;
+  if (t0 >= tiles) return;
+  // Tiles by the length of their sums, the longer half first and the rest from the
+  // shortest up: workgroups that share a CU come half a launch apart (n = 3000, f64:
+  // the last level's first product 197 -> 131 us, its second 76 -> 64, against row
+  // order, in which the longest shared one).
+  if (t0 >= half) t0 = tiles - 1 - (t0 - half);
+  const int m0 = (FIRST ? t0 % mt : mt - 1 - t0 / nt) * 64, n0 = (FIRST ? t0 / mt : t0 % nt) * 64;
   T* t = tmp + (int64_t)blockIdx.y * h * h;
   const T* w = W + (int64_t)o * ldw + o;
   typename Mfma<T>::acc_t acc[2];
