@@ -479,8 +479,10 @@ TRAFFIC_FILE = os.path.join(ROOT, "profiles", "trailing_syrk_f64_n32768_traffic.
 
 
 def _is_trailing_syrk(name):
-    # the square lower-triangle instantiation (TRI, SQ) of the NT MFMA kernel
-    return name.startswith("void llh::(anonymous namespace)::gemm_nt_kernel<double,") and ", true, true, " in name
+    # the square lower-triangle instantiations (TRI, SQ) of the NT MFMA kernels
+    pre = "void llh::(anonymous namespace)::"
+    return (name.startswith(pre + "nt_dma_kernel<double, true, true>") or
+            name.startswith(pre + "gemm_nt_kernel<double,") and ", true, true, " in name)
 
 
 def rocprof_summary(trace_dir, fetch_dir, write_dir, n, out_md, out_json, command):
@@ -525,7 +527,7 @@ def rocprof_summary(trace_dir, fetch_dir, write_dir, n, out_md, out_json, comman
             alg.append(8.0 * (m3 * (m3 + 1) + m3 * kb))
         k0 += kb
     alg_avg = sum(alg) / len(alg)
-    res = {"n": n, "kernel_class": "trailing SYRK (gemm_nt_kernel<double,...,TRI,SQ>)",
+    res = {"n": n, "kernel_class": "trailing SYRK (nt_dma_kernel<double,TRI,SQ>)",
            "avg_launch_us": syrk_ns / syrk_calls / 1e3, "launches": syrk_calls,
            "fetch": counters["FETCH_SIZE"], "write": counters["WRITE_SIZE"],
            "traffic_bytes_per_launch": traffic, "algorithmic_bytes_per_launch": alg_avg,
@@ -543,9 +545,8 @@ def rocprof_summary(trace_dir, fetch_dir, write_dir, n, out_md, out_json, comman
             short = short[:87] + "..."
         lines.append(f"| `{short}` | {r['Calls']} | {float(r['AverageNs']) / 1e3:.1f} | "
                      f"{float(r['TotalDurationNs']) / 1e6:.1f} | {float(r['Percentage']):.1f} |")
-    lines += ["", f"Trailing SYRK (the TRI+SQ instantiations of `gemm_nt_kernel`, launched only by "
-                  f"`launch_syrk_lower`: 256x128 tiles while the trailing matrix is at least 4096^2, 128x128 "
-                  f"below): {syrk_calls} launches, average {syrk_ns / syrk_calls / 1e3:.1f} us per launch.", "",
+    lines += ["", f"Trailing SYRK (the TRI+SQ instantiation of `nt_dma_kernel`, launched only by "
+                  f"`launch_syrk_lower`: 128x128 tiles): {syrk_calls} launches, average {syrk_ns / syrk_calls / 1e3:.1f} us per launch.", "",
               "## HBM traffic per trailing-SYRK launch (`--pmc FETCH_SIZE`, then `--pmc WRITE_SIZE`)", "",
               "| counter | copy of A reads (KiB) | known (KiB) | factor | avg per launch (KiB) | bytes per launch |",
               "|---|---:|---:|---:|---:|---:|"]
@@ -839,8 +840,7 @@ def main():
                                  "a copy of A), %.2fx the algorithmic bytes; profiles/trailing_syrk_f64_n%d.md"
                                  % (tr["fetch"]["factor"], tr["write"]["factor"], tr["traffic_over_algorithmic"], n))
                 if tr else None,
-                "kernel": "gemm_nt_kernel<double,256,128,4,2,TRI,SQ> (trailing SYRK, rank %d; 128x128 tiles once the "
-                          "trailing matrix is below 4096^2)" % outer_width(n),
+                "kernel": "nt_dma_kernel<double,TRI,SQ> (trailing SYRK, rank %d; 128x128 tiles)" % outer_width(n),
                 "avg_launch_us": round(tot_ms / cnt * 1e3, 2), "launches_per_step": cnt // args.steps,
                 "algorithmic_tflop_per_step": round(fl / args.steps / 1e12, 4)}
 

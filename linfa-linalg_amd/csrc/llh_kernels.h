@@ -204,10 +204,6 @@ hipError_t launch_gemm_nt_h(bool tri, int M, int N, int K, float alpha, const _F
                                 const _Float16* B, int64_t ldb, float beta, float* C, int64_t ldc,
                                 const int32_t* gate, hipStream_t s);
 
-// k_trsm.hip: panel solve X := X * L^-T (X is m x b, L is b x b lower, b <= kNB).
-template <typename T>
-hipError_t launch_trsm_rows(int m, int b, T* X, int64_t ldx, const T* L, int64_t ldl, const int32_t* gate,
-                            hipStream_t s);
 // k_trsm.hip: diagonal-block solve op(T) Y = Y for b <= kNB rows and m columns
 // of a row-major Y; upper_op selects back substitution; trans reads T^T.
 template <typename T>
