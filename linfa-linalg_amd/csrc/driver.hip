@@ -237,7 +237,7 @@ hipError_t trsm_split(bool upper_op, bool trans, int n, const T* a, int64_t lda,
                       const int32_t* gate) {
   const double es = (double)sizeof(T);
   if (n <= solve_split<T>(m)) {
-    // the launcher resets the ticket; the error word is the call's (solve_sync_begin)
+    // the launch leaves the ticket at 0; the error word is the call's (solve_sync_begin)
     const int most = (int)std::min<int64_t>(sync->nmail * kSolveChunkHost, INT_MAX);
     for (int c = 0; c < m; c += most) {
       const int mc = std::min(most, m - c);

@@ -106,8 +106,9 @@ __global__ __launch_bounds__(256) void trtri64_kernel(int n, const TS* __restric
 // trsm_persistent: op(A) X = B in place for up to kSolveChunk right-hand-side
 // columns per workgroup, one launch for the whole solve.
 //
-// Workgroups take tickets in launch order; ticket t is (position p, column chunk
-// q).  Position p is block row w = p (forward, op(A) lower) or w = nb-1-p
+// Workgroups take tickets in launch order, every one of them, and the last sets the
+// counter back (a launch of its own for that cost 5 us a solve); ticket t is (position
+// p, column chunk q).  Position p is block row w = p (forward, op(A) lower) or w = nb-1-p
 // (backward).  The workgroup accumulates sum_j op(A)_wj X_j over the blocks j
 // that precede w in solve order, then forms X_w = inv(op(A)_ww) (B_w - sum) with
 // the precomputed inverse and publishes it.  A workgroup only ever waits for
@@ -173,12 +174,11 @@ __device__ __forceinline__ void agent_store(T* p, T v) {
                        __HIP_MEMORY_SCOPE_AGENT);
 }
 
-template <typename T, bool VEC>
+template <typename T, bool VEC, bool trans>
 __global__ __launch_bounds__(256, 2) void trsm_persistent_kernel(
-    int n, int m, const T* __restrict__ A, int64_t lda, bool trans, bool lower_op, const T* __restrict__ Dinv,
+    int n, int m, const T* __restrict__ A, int64_t lda, bool lower_op, const T* __restrict__ Dinv,
     bool dinv_t, T* B, int64_t ldb, int32_t* ticket, int32_t* flags, uint64_t* mail, int32_t epoch, int32_t* err,
     int64_t spin_limit, const int32_t* __restrict__ gate) {
-  if (gate != nullptr && *gate != kNoFail) return;
   using MF = Mfma<T>;
   using acc_t = typename MF::acc_t;
   // kFar (f64): G_2 waits in LDS, since with both in registers some are spilled (3.6 us
@@ -199,7 +199,9 @@ __global__ __launch_bounds__(256, 2) void trsm_persistent_kernel(
   if (tid < 3) s_abort[tid] = 0;
   __syncthreads();
   const int tk = __builtin_amdgcn_readfirstlane(s_ticket);
-  if (tk >= nb * nq) return;
+  // (the last ticket: no workgroup takes another one, the next launch starts at 0)
+  if (tk == nb * nq - 1 && tid == 0) atomicExch(ticket, 0);
+  if (gate != nullptr && *gate != kNoFail) return;
   const int p = tk / nq, q = tk % nq;
   const int w = lower_op ? p : nb - 1 - p;
   const int w0 = w * kNB, bw = min(kNB, n - w0);
@@ -262,14 +264,33 @@ __global__ __launch_bounds__(256, 2) void trsm_persistent_kernel(
     for (int e = 0; e < NK; ++e) far[64 * e] = g2[e];
   }
 
-  // this lane's values of op(A)[w0 + 16 i + fr, j0 + 16 wv + 4 fq + e], at 4 i + e
+  // The row of block w that MFMA row f of row tile i stands for: for op(A) = A^T a lane's
+  // rows of the tiles lie side by side in memory (16-byte loads; n = 12000, m = 16 f64 3.9 -> 2.5 us a
+  // hop, f32 2.8 -> 2.0).
+  auto arow = [&](int i, int f) __attribute__((always_inline)) {
+    constexpr int V = 16 / (int)sizeof(T);
+    return trans ? i / V * 16 * V + f * V + i % V : 16 * i + f;
+  };
+  // this lane's values of op(A)[w0 + arow(i, fr), j0 + 16 wv + 4 fq + e], at 4 i + e
   typedef T vec_t __attribute__((ext_vector_type(16 / sizeof(T))));
   constexpr int VL = 16 / sizeof(T);
   auto fetch = [&](int st, T (&out)[NK]) __attribute__((always_inline)) {
     const int j0 = jof(st) * kNB, bj = min(kNB, n - j0), k0 = 16 * wv + 4 * fq;
+    if (trans && VEC && bj == kNB && bw == kNB) {
+      const T* col = A + (int64_t)(j0 + k0) * lda + w0 + VL * fr;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int v = 0; v < 4 / VL; ++v) {
+          const vec_t x = *reinterpret_cast<const vec_t*>(col + (int64_t)e * lda + 16 * VL * v);
+#pragma unroll
+          for (int c = 0; c < VL; ++c) out[4 * (VL * v + c) + e] = x[c];
+        }
+      return;
+    }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const int64_t r = w0 + min(16 * i + fr, bw - 1);
+      const int64_t r = w0 + min(arow(i, fr), bw - 1);
       if (!trans) {
         const T* row = A + r * lda + j0 + k0;
         if (VEC && bj == kNB) {
@@ -395,7 +416,7 @@ __global__ __launch_bounds__(256, 2) void trsm_persistent_kernel(
 #pragma unroll
   for (int i = 0; i < 4; ++i)
 #pragma unroll
-    for (int e = 0; e < 4; ++e) Wk[wv * SL + sidx(16 * i + MF::row(lane, e), fr)] = acc[i][e];
+    for (int e = 0; e < 4; ++e) Wk[wv * SL + sidx(arow(i, MF::row(lane, e)), fr)] = acc[i][e];
   __syncthreads();
   if (s_abort[0]) return;
 #pragma unroll
@@ -499,15 +520,18 @@ hipError_t launch_trsm_persistent(int n, int m, const T* A, int64_t lda, bool tr
                                   int64_t spin_limit, const int32_t* gate, hipStream_t s) {
   if (n <= 0 || m <= 0) return hipSuccess;
   const int nb = (n + kNB - 1) / kNB, nq = (m + kSolveChunk - 1) / kSolveChunk;
-  hipError_t e = launch_fill_i32(ticket, 0, 1, s);
-  if (e != hipSuccess) return e;
   const bool vec = (reinterpret_cast<uintptr_t>(A) % 16 == 0) && ((lda * sizeof(T)) % 16 == 0);
-  if (vec)
-    hipLaunchKernelGGL((trsm_persistent_kernel<T, true>), dim3(nb * nq), dim3(256), 0, s, n, m, A, lda, trans,
-                       lower_op, Dinv, dinv_t, B, ldb, ticket, flags, mail, epoch, err, spin_limit, gate);
-  else
-    hipLaunchKernelGGL((trsm_persistent_kernel<T, false>), dim3(nb * nq), dim3(256), 0, s, n, m, A, lda, trans,
-                       lower_op, Dinv, dinv_t, B, ldb, ticket, flags, mail, epoch, err, spin_limit, gate);
+#define LLH_TRSM_GO(VEC, TRANS)                                                                                   \
+  hipLaunchKernelGGL((trsm_persistent_kernel<T, VEC, TRANS>), dim3(nb * nq), dim3(256), 0, s, n, m, A, lda, lower_op, \
+                     Dinv, dinv_t, B, ldb, ticket, flags, mail, epoch, err, spin_limit, gate)
+  if (vec) {
+    if (trans) LLH_TRSM_GO(true, true);
+    else LLH_TRSM_GO(true, false);
+  } else {
+    if (trans) LLH_TRSM_GO(false, true);
+    else LLH_TRSM_GO(false, false);
+  }
+#undef LLH_TRSM_GO
   return hipGetLastError();
 }
 
