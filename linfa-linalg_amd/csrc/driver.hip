@@ -114,11 +114,11 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
   // bytes per panel element of the trailing update (the f16 copy is written
   // and read once more)
   const double pes = half != nullptr ? es + 4.0 : es;
-  LLH_TRY(launch_fill_i32(info, kNoFail, 1, s));
+  if (n > small_max<T>() && dinv == nullptr) return hipErrorInvalidValue;  // the blocked path needs the inverses
+  if (n <= 0 || n > small_max<T>()) LLH_TRY(launch_fill_i32(info, kNoFail, 1, s));
   if (n <= 0) return hipSuccess;
-  if (n <= small_max<T>() || dinv == nullptr) {
-    if (n > small_max<T>()) return hipErrorInvalidValue;  // the blocked path needs the inverse buffer
-    LLH_TRY(launch_potrf_exact_single<T>(a, lda, n, info, 0, nullptr, s));
+  if (n <= small_max<T>()) {
+    LLH_TRY(launch_potrf_exact_single<T>(a, lda, n, info, zero_upper, s));
     if (dinv != nullptr) LLH_TRY(launch_trtri_blocks<T>(n, a, lda, false, false, dinv, info, s));
   } else {
     const int kb0 = std::min(panel_width(n, n, half != nullptr), n);
@@ -222,7 +222,7 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
       LLH_TRY(hipStreamWaitEvent(s, la->fwd_ev, 0));
     }
   }
-  if (zero_upper) LLH_TRY(launch_zero_triangle<T>(a, lda, n, true, info, s));
+  if (zero_upper && n > small_max<T>()) LLH_TRY(launch_zero_triangle<T>(a, lda, n, true, info, s));
   return hipSuccess;
 }
 

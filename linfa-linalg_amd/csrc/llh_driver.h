@@ -86,8 +86,9 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
 // Enqueues op(A) X = B in place (B row-major n x m); upper_op names the triangle
 // of op(A) and trans != 0 means op(A) = A^T.  dinv, when non-null, holds the
 // inverses of op(A)'s 64 x 64 diagonal blocks (transposed when dinv_t);
-// otherwise they are computed into dinv_work.  With sync and m <= 64 the solve
-// is one persistent launch; otherwise it is a sequence of blocked launches.
+// otherwise they are computed into dinv_work.  With sync the solve is
+// one persistent launch for m <= 64 and a few with products between beyond that
+// (solve_split); otherwise it is a sequence of blocked launches.
 // gate (optional): the factor's status word; once it holds a failed row every
 // kernel of the solve is a no-op and B keeps its values.
 template <typename T>

@@ -73,12 +73,11 @@ constexpr int small_max() { return sizeof(T) == 8 ? kSmallMaxD : kSmallMaxS; }
 template <typename T>
 struct small_max_c { static constexpr int value = small_max<T>(); };
 
-// k_small.hip: exact-order LDS Cholesky (bit-identical to the reference order).
-// TS is the storage type, T the arithmetic type (T = TS except for the f64
-// diagonal blocks of the mixed-precision factor).
-template <typename TS, typename T = TS>
-hipError_t launch_potrf_exact_single(TS* a, int64_t lda, int n, int32_t* info, int64_t info_base,
-                                     const int32_t* gate, hipStream_t s);
+// k_small.hip: exact-order Cholesky of one matrix, n <= small_max<T>() (bit-identical to
+// the reference order).  *info receives kNoFail or the first failing row; zero_upper
+// zeroes the strict upper triangle where none fails.
+template <typename T>
+hipError_t launch_potrf_exact_single(T* a, int64_t lda, int n, int32_t* info, bool zero_upper, hipStream_t s);
 template <typename T>
 hipError_t launch_potrf_potrs_exact_batched(const SmallDesc<T>* descs, int count, int nmax, int do_solve,
                                             hipStream_t s);
