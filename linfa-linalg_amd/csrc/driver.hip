@@ -241,6 +241,13 @@ hipError_t trsm_split(bool upper_op, bool trans, int n, const T* a, int64_t lda,
     const int most = (int)std::min<int64_t>(sync->nmail * kSolveChunkHost, INT_MAX);
     for (int c = 0; c < m; c += most) {
       const int mc = std::min(most, m - c);
+      // (before the values run out the words are cleared and they start anew: some 20
+      // hours of solves without a pause)
+      if (*sync->epoch > INT_MAX - solve_epochs(n)) {
+        LLH_TRY(launch_fill_i32(sync->words + 2, 0, sync->nflags, s));
+        LLH_TRY(launch_fill_i32(reinterpret_cast<int32_t*>(sync->mail), 0, 2 * solve_mail_words(sync->nmail), s));
+        *sync->epoch = 1;
+      }
       const int32_t epoch = *sync->epoch;
       *sync->epoch += solve_epochs(n);
       const double fl = (double)n * n * mc;

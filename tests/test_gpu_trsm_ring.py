@@ -43,3 +43,27 @@ def test_solves_in_turn(dtype):
     """Larger and smaller solves in one context: no block of an earlier one is taken."""
     for i, (n, m) in enumerate([(1300, 16), (600, 40), (1300, 16), (200, 16), (700, 100), (1300, 1)]):
         _check(n, m, dtype, i % 2 == 0, i % 3 == 0, i)
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+def test_epochs_start_anew(dtype):
+    """The solves before and after the context's epochs run out (set from here: the
+    member in front of the spin limit, found by a value of that)."""
+    import ctypes
+
+    from linfa_linalg_hip import device as dev
+    _check(600, 40, dtype, False, False, 1)  # the buffers exist
+    h = dev.context().handle
+    base = h.value if isinstance(h, ctypes.c_void_p) else int(h)
+    mark = 0x5A3C1D97E
+    dev.set_solve_spin_limit(mark)
+    try:
+        at = next(o for o in range(8, 2048, 8) if ctypes.c_int64.from_address(base + o).value == mark)
+    finally:
+        dev.set_solve_spin_limit(0)
+    epoch = ctypes.c_int32.from_address(base + at - 8)
+    assert 1 < epoch.value < 1 << 30
+    epoch.value = 2 ** 31 - 4
+    for i in range(4):
+        _check(600, 40, dtype, i % 2 == 1, False, i)  # two epochs each
+    assert epoch.value < 100
