@@ -160,7 +160,6 @@ hipError_t ctx_sync(llh_context* ctx, int n, int m, SolveSync* sync) {
   sync->nflags = (int64_t)(ctx->sync.bytes / sizeof(int32_t)) - 2;
   sync->epoch = &ctx->epoch;
   sync->spin_limit = ctx->spin_limit;
-  sync->wild = ctx->d_info + 1;
   // one error word per call: cleared here, read back once the call's sweeps are done
   return solve_sync_begin(*sync, ctx->stream);
 }
@@ -177,16 +176,6 @@ hipError_t ctx_read_solve_error(llh_context* ctx) {
 }  // namespace llh
 
 namespace {
-
-// Whether a triangular solve of m columns left B untouched because a diagonal
-// block's inverse is not to be used (trsm_enqueue); the context's stream has been
-// waited for, ctx->h_info[1] read with ctx_read_solve_wild.
-bool solve_wild(const llh_context* ctx, size_t m) { return m > 64 && ctx->h_info[1] != kNoFail; }
-hipError_t ctx_read_solve_wild(llh_context* ctx, size_t m) {
-  ctx->h_info[1] = kNoFail;
-  if (m <= 64 || m > (size_t)kSolveMaxCols) return hipSuccess;
-  return hipMemcpyAsync(ctx->h_info + 1, ctx->d_info + 1, sizeof(int32_t), hipMemcpyDeviceToHost, ctx->stream);
-}
 
 llh_status solve_stalled(llh_error* err) {
   return set_error(err, LLH_ERR_HIP, 0, 0, -1, "triangular solve: a block wait exceeded its bound", 0);
@@ -418,18 +407,10 @@ llh_status solve_triangular_plain(llh_context* ctx, size_t rows, size_t cols, co
                             ctx->profiler()),
             "trsm");
   CHECK_HIP(ctx_read_solve_error(ctx), "solve status");
-  CHECK_HIP(ctx_read_solve_wild(ctx, b_cols), "solve status");
   CHECK_HIP(hipMemcpyAsync(hb, db, n * b_cols * sizeof(T), hipMemcpyDeviceToHost, ctx->stream),
             "download");
   CHECK_HIP(hipStreamSynchronize(ctx->stream), "synchronize");
   if (ctx->h_info[2] != 0) return solve_stalled(err);
-  if (solve_wild(ctx, b_cols)) {
-    CHECK_HIP(trsm_enqueue<T>(uplo == LLH_UPPER, false, (int)n, da, (int64_t)n, (int)b_cols, db, (int64_t)b_cols,
-                              nullptr, false, nullptr, nullptr, ctx->stream, ctx->profiler()),
-              "trsm");
-    CHECK_HIP(hipMemcpyAsync(hb, db, n * b_cols * sizeof(T), hipMemcpyDeviceToHost, ctx->stream), "download");
-    CHECK_HIP(hipStreamSynchronize(ctx->stream), "synchronize");
-  }
   scatter(hb, n, b_cols, b, brs, bcs, [b_cols](size_t) { return b_cols; });
   return ok(err);
 }
@@ -607,15 +588,8 @@ llh_status dev_solve_triangular(llh_context* ctx, llh_uplo uplo, int trans, size
                             nullptr, false, static_cast<T*>(dinv), &sync, ctx->stream, ctx->profiler()),
             "trsm");
   CHECK_HIP(ctx_read_solve_error(ctx), "solve status");
-  CHECK_HIP(ctx_read_solve_wild(ctx, m), "solve status");
   CHECK_HIP(hipStreamSynchronize(ctx->stream), "synchronize");
   if (ctx->h_info[2] != 0) return solve_stalled(err);
-  if (solve_wild(ctx, m)) {
-    CHECK_HIP(trsm_enqueue<T>(uplo == LLH_UPPER, trans != 0, (int)n, a, (int64_t)lda, (int)m, b, (int64_t)ldb,
-                              nullptr, false, nullptr, nullptr, ctx->stream, ctx->profiler()),
-              "trsm");
-    CHECK_HIP(hipStreamSynchronize(ctx->stream), "synchronize");
-  }
   return ok(err);
 }
 
@@ -766,7 +740,6 @@ llh_status dev_apply_constraints(llh_context* ctx, size_t n, size_t k, T* v, siz
   CHECK_HIP(ctx_dinv(ctx, KY, sizeof(T), &dv), "inverse buffer");
   SolveSync sync;
   CHECK_HIP(ctx_sync(ctx, KY, K, &sync), "solve sync");
-  sync.wild = nullptr;  // (its answer is not waited for here: k > 64 solves by substitution)
   CHECK_HIP(trsm_enqueue<T>(false, false, KY, l_yy, (int64_t)ldl, K, g, (int64_t)K, nullptr, false,
                             static_cast<T*>(dv), &sync, s, ctx->profiler()),
             "solve");

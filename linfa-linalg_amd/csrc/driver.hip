@@ -228,9 +228,9 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
 
 namespace {
 
-// op(A) X = B with the inverses of the diagonal blocks: one launch
-// (launch_trsm_persistent) up to solve_split<T>(m) rows, otherwise by halves: the
-// half that comes first, one product into the other half's rows, the other half.
+// op(A) X = B with the inverses of the diagonal blocks, or by substitution (dinv
+// null): one launch (launch_trsm_persistent) up to solve_split<T>(m) rows, otherwise by
+// halves: the half that comes first, one product into the other half's rows, the other half.
 template <typename T>
 hipError_t trsm_split(bool upper_op, bool trans, int n, const T* a, int64_t lda, int m, T* b, int64_t ldb,
                       const T* dinv, bool dinv_t, SolveSync* sync, hipStream_t s, Profiler* prof,
@@ -260,7 +260,7 @@ hipError_t trsm_split(bool upper_op, bool trans, int n, const T* a, int64_t lda,
     return hipSuccess;
   }
   const int n1 = ((n + kNB - 1) / kNB + 1) / 2 * kNB, n2 = n - n1;
-  const T* d2 = dinv + (int64_t)(n1 / kNB) * kNB * kNB;
+  const T* d2 = dinv == nullptr ? nullptr : dinv + (int64_t)(n1 / kNB) * kNB * kNB;
   const T* a22 = a + (int64_t)n1 * lda + n1;
   T* b2 = b + (int64_t)n1 * ldb;
   const double fl = 2.0 * n1 * n2 * m, by = es * ((double)n1 * n2 + 2.0 * n * m);
@@ -290,21 +290,14 @@ hipError_t trsm_enqueue(bool upper_op, bool trans, int n, const T* a, int64_t ld
                         Profiler* prof, const int32_t* gate) {
   if (n <= 0 || m <= 0) return hipSuccess;
   const double es = (double)sizeof(T);
+  const bool inverses = m <= 64;
   if (sync != nullptr && sync->epoch != nullptr && m <= kSolveMaxCols && sync->nflags >= solve_flags<T>(n, m) &&
-      sync->mail != nullptr && sync->nmail > 0 &&
-      (dinv != nullptr || (dinv_work != nullptr && (m <= 64 || sync->wild != nullptr)))) {
-    if (dinv == nullptr) {
-      // Above 64 columns the caller looks at *wild afterwards and, where a
-      // diagonal block is singular or its inverse large, takes the substitution
-      // below instead (this path then leaves B untouched).
-      int32_t* wild = m > 64 ? sync->wild : nullptr;
-      if (wild != nullptr) {
-        if (gate != nullptr) return hipErrorInvalidValue;
-        LLH_TRY(launch_fill_i32(wild, kNoFail, 1, s));
-        gate = wild;
-      }
+      sync->mail != nullptr && sync->nmail > 0 && (!inverses || dinv != nullptr || dinv_work != nullptr)) {
+    if (!inverses) {
+      dinv = nullptr;
+    } else if (dinv == nullptr) {
       LLH_PROF(kSolveDiag, (double)n * kNB * kNB / 3.0, es * (double)n * kNB,
-               (launch_trtri_blocks<T>(n, a, lda, trans, upper_op, dinv_work, nullptr, s, wild)));
+               (launch_trtri_blocks<T>(n, a, lda, trans, upper_op, dinv_work, gate, s)));
       dinv = dinv_work;
       dinv_t = false;
     }

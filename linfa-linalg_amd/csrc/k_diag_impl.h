@@ -40,15 +40,6 @@
 
 namespace llh {
 
-
-// Calls f(std::integral_constant<int, I>) for I = 0 .. n-1: the panel loops are
-// expanded at compile time, so every index into the register arrays is a
-// constant (a rolled loop would move them to scratch memory).
-template <typename F, int... I>
-__device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F&& f) {
-  (f(std::integral_constant<int, I>{}), ...);
-}
-
 // The instructions of a sweep's column, as blocks of volatile asm that issue in
 // the order given.  row_newbcast:Q is the DPP broadcast of lane Q of each group of
 // 16 lanes; the compiler would split a broadcast FMA into a move and a dependent

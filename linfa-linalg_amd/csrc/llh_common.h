@@ -5,6 +5,8 @@
 
 #include <cstddef>
 #include <cstdint>
+#include <type_traits>
+#include <utility>
 
 namespace llh {
 
@@ -66,11 +68,11 @@ inline int solve_epochs(int n) { return ((n + kNB - 1) / kNB + kMailRing - 1) / 
 // (trsm_split): all of them up to 64 columns, where the chain of 64-row hops
 // bounds it; with more columns n * m = 6M, about as many as keep its products
 // shorter than that chain, the rest as products with larger tiles between launches.
-// Measured (us, L / L^T) at 1.5M / 3M / 6M / 12M: f64 n = 4096 m = 1500 1494, 1460 / 1192,
-// 1185 / 1069, 1116 / -, n = 12000 m = 500 3707, 3663 / 2909, 3110 / 2562, 3091 / -; f32
-// n = 4096 m = 1500 942, 1001 / 804, 827 / 705, 757 / 707, 840, n = 12000 m = 500
-// 2325, 2451 / 1900, 2047 / 1654, 1924 / 1709, 2312; m = 1500 4698 / 4258 / 4081 / 3977,
-// 4746 / 4301 / 4338 / 4721.
+// Measured (us, L / L^T) at 1.5M, 3M, 6M, 12M: f64 n = 4096 m = 1500 1393 / 1347, 1116 /
+// 1047, 957 / 885, 1001 / 925, n = 12000 m = 500 3730 / 3560, 2894 / 2800, 2462 / 2380,
+// 2622 / 2579; f32 n = 4096 m = 1500 892 / 932, 765 / 747, 690 / 592, 678 / 541, n = 12000
+// m = 500 2391 / 2427, 1916 / 1921, 1630 / 1512, 1995 / 1433, m = 1500 4622 / 4568, 4298 /
+// 4016, 4133 / 3701, 3901 / 3419.
 constexpr int kSolveMaxCols = 32768;
 template <typename T>
 inline int solve_split(int m) {
@@ -101,5 +103,13 @@ template <>
 __device__ __forceinline__ double sqrt_rn<double>(double a) { return __builtin_sqrt(a); }
 template <>
 __device__ __forceinline__ float sqrt_rn<float>(float a) { return __builtin_sqrtf(a); }
+
+// Calls f(std::integral_constant<int, I>) for I = 0 .. n-1: loops are
+// expanded at compile time, so every index into the register arrays is a
+// constant (a rolled loop would move them to scratch memory).
+template <typename F, int... I>
+__device__ __forceinline__ void static_for(std::integer_sequence<int, I...>, F&& f) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
 
 }  // namespace llh

@@ -21,9 +21,6 @@ struct SolveSync {
   int64_t nmail = 0;  // 16-column chunks that mail has room for
   int32_t* epoch = nullptr;
   int64_t spin_limit = kSpinLimit;  // bound on each flag wait (negative: give up at once)
-  // Device word of solves of more than 64 columns with inverses of their own
-  // (trsm_enqueue): kNoFail, or a diagonal block whose inverse is not to be used.
-  int32_t* wild = nullptr;
 };
 
 // Enqueues the clearing of the solve error word: once per call, before its
@@ -84,9 +81,10 @@ hipError_t potrf_enqueue(T* a, int64_t lda, int n, int32_t* info, bool zero_uppe
                          _Float16* half = nullptr, const FwdFuse<T>* ff = nullptr);
 
 // Enqueues op(A) X = B in place (B row-major n x m); upper_op names the triangle
-// of op(A) and trans != 0 means op(A) = A^T.  dinv, when non-null, holds the
-// inverses of op(A)'s 64 x 64 diagonal blocks (transposed when dinv_t);
-// otherwise they are computed into dinv_work.  With sync the solve is
+// of op(A) and trans != 0 means op(A) = A^T.  Up to 64 columns it multiplies by the
+// inverses of op(A)'s 64 x 64 diagonal blocks: dinv where it is non-null (transposed when
+// dinv_t), otherwise they are computed into dinv_work.  More columns are solved by
+// substitution, which needs neither.  With sync the solve is
 // one persistent launch for m <= 64 and a few with products between beyond that
 // (solve_split); otherwise it is a sequence of blocked launches.
 // gate (optional): the factor's status word; once it holds a failed row every

@@ -213,9 +213,10 @@ hipError_t launch_trsv_block(bool upper_op, bool trans, int b, const T* Tm, int6
 // as consecutive row-major 64 x 64 blocks at out; upper names op(A)'s triangle.
 template <typename TS, typename T = TS>
 hipError_t launch_trtri_blocks(int n, const TS* A, int64_t lda, bool trans, bool upper, TS* out,
-                               const int32_t* gate, hipStream_t s, int32_t* wild = nullptr);
+                               const int32_t* gate, hipStream_t s);
 // k_trsm.hip: one-launch blocked solve op(A) X = B (B row-major n x m) using the
-// diagonal-block inverses Dinv (transposed when dinv_t).  ticket/flags/err are
+// diagonal-block inverses Dinv (transposed when dinv_t), or substituting in the diagonal
+// blocks with Dinv null.  ticket/flags/err are
 // device words (ticket: 0 before the first launch; flags: one per 64-row block and 16-column chunk), mail holds
 // solve_mail_words(1) zeroed words per 16-column chunk, and epoch .. epoch +
 // solve_epochs(n) - 1 are values that neither has ever held.  *err becomes non-zero if a wait exceeded spin_limit
