@@ -8,6 +8,7 @@
 #include "llh_kernels.h"
 #include "k_gemm_impl.h"
 #include "k_trsm_impl.h"
+#include "llh_wait.h"
 
 #include <type_traits>
 #include <utility>
@@ -136,7 +137,8 @@ __global__ __launch_bounds__(256) void trtri64_kernel(int n, const TS* __restric
 // A negative spin_limit makes every wait give up at once (a host-forced failure
 // for tests of the error path; every workgroup still exits normally).  With a
 // gate (the factor's status word) that holds a failed row, every workgroup
-// returns at once and B is left untouched.
+// returns at once and B is left untouched; where the gate is set while the launch runs,
+// the waits end on it too, without an error (wait_step), and B may be partly solved.
 constexpr int kSolveChunk = kSolveChunkHost;
 constexpr int kFlagWindow = 64;  // flags checked ahead per wait
 constexpr int kMailReach = 4;    // positions that read a block from the ring
@@ -353,13 +355,14 @@ __global__ __launch_bounds__(256, 2) void trsm_persistent_kernel(
     for (int e = 0; e < 4; ++e)
       out[e] = (k0 + e < bj && fr < mc) ? agent_load(&B[(int64_t)(j0 + k0 + e) * ldb + c0 + fr]) : T(0);
   };
-  // one more poll of a wait: false once it gives up
+  // one more poll of a wait: false once it gives up or leaves
   auto go_on = [&](int64_t& it, int stage) -> bool {
-    if (spin_limit >= 0 && ++it <= spin_limit &&
-        ((it & 7) != 0 || __hip_atomic_load(err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0))
-      return true;
+    const Wait next = wait_step(
+        it, spin_limit, kNoFail, [&] { return agent_load(err); },
+        [&] { return gate != nullptr ? agent_load(gate) : kNoFail; });
+    if (next == Wait::kGoOn) return true;
     if (lane == 0) {
-      atomicExch(err, 1);
+      if (next == Wait::kGiveUp) atomicExch(err, 1);
       s_abort[stage] = 1;
     }
     return false;
