@@ -21,7 +21,7 @@ union StepLds {
     TS lk[kNB * step_ls<TS>()];  // L(k, k-1)
     T conv[4][sizeof(TS) == sizeof(T) ? 1 : diag_blk<T>()];  // a block's change of layout, one per wave
     int fail[kNB / kDiagW];
-    int skip;
+    int status;
   } c;
   struct {
     NtSlab<TS, 64> as[2];
@@ -37,10 +37,13 @@ union StepLds {
 // no workgroup waits for another one and the step is one launch instead of
 // three; beside the sweeps it applies column k - 1 to its own 64 rows (held
 // transposed, in registers) and multiplies them by each column block of the inverse
-// once the sweep has it.  Workgroup 0 also stores the inverse (dinv slot k) and L_kk.
-// The other workgroups still read the block that L_kk replaces, so L_kk waits in the
-// next inverse's slot until launch k + 1 copies it (the launch without rows below
-// stores it directly).
+// once the sweep has it.  Workgroup 0 also stores the inverse (dinv slot k) and L_kk, and
+// the status of a failing pivot.  The other workgroups, some of which may start late, still
+// read the block that L_kk replaces: L_kk, or what a failing block has of it, waits in
+// the next inverse's slot until launch k + 1 copies it (the launch without rows below
+// stores it directly).  For the same reason a launch looks at failures before its own
+// block only: every workgroup of the launch that fails finds the block and the status as
+// they were and does the same, whenever it runs.
 // Update workgroups (the rest): apply column k - 1 to the panel's later columns,
 // one 64 x 64 tile each.
 //
@@ -67,7 +70,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, 2) void panel_step_kernel(TS* a, 
   const bool prev = k0 > p0;
   const int r0 = k0 + kNB;  // first row below the diagonal block
   if ((int)blockIdx.x >= nchain) {
-    if (*info != kNoFail) return;
+    if (*info < k0) return;
     const int u = blockIdx.x - nchain, ri = u / ncol, jj = u % ncol;
     if (jj > ri) return;
     const TS* p = a + (int64_t)r0 * lda + (k0 - kNB);
@@ -85,7 +88,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, 2) void panel_step_kernel(TS* a, 
   const bool factor = !WIDE || wv < NS, solver = !WIDE || wv >= NS;
   const int b = min(kNB, n - k0);
   const bool rows = r0 < n, first = blockIdx.x == 0;
-  if (tid == 0) sm.c.skip = *info != kNoFail;
+  if (tid == 0) sm.c.status = *info;
   TS* const slot = dinv + (int64_t)(k0 / kNB) * kNB * kNB;
   TS* const akk = a + (int64_t)k0 * lda + k0;
 
@@ -132,16 +135,19 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, 2) void panel_step_kernel(TS* a, 
     for (int e = 0; e < kNB * kNB / NT; ++e) lprev[e] = slot[tid + NT * e];
   }
   diag_barrier();
-  if (sm.c.skip) return;
+  const int status = sm.c.status;
   if (copy && first) {
-    // L_(k-1)(k-1) from this block's slot, read above, to its place
+    // L_(k-1)(k-1) from this block's slot, read above, to its place; of a block that failed
+    // at row `last` the rows before it and L[last, ..last] (an earlier failure: nothing)
+    const int last = status < k0 ? status - (k0 - kNB) : kNB;
     TS* dst = a + (int64_t)(k0 - kNB) * lda + (k0 - kNB);
 #pragma unroll
     for (int e = 0; e < kNB * kNB / NT; ++e) {
       const int idx = tid + NT * e, row = idx / kNB, col = idx % kNB;
-      if (col <= row) dst[(int64_t)row * lda + col] = lprev[e];
+      if (row < last ? col <= row : row == last && col < row) dst[(int64_t)row * lda + col] = lprev[e];
     }
   }
+  if (status < k0) return;
 
   // L(k, k-1)'s strip c times this wave's strip (!left) or the transposed rows (left),
   // added to x, summed by itself first: added term by term, every partial sum would
@@ -210,14 +216,8 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, 2) void panel_step_kernel(TS* a, 
   const int fail = diag_core<T, WIDE>(
       tacc, wv, sm.c.l, sm.c.fail,
       [&](int w, int it, int f) __attribute__((always_inline)) {
-        if (!first) return;
-        // L_kk beside the block while others may read it; a failing block's rows
-        // go to their place (nothing after this launch reads the block)
-        if (f >= 0) {
-          diag_put<TS, T>(sm.c.l, w, it, f, b, akk, lda, slot);
-        } else {
-          diag_put<TS, T>(sm.c.l, w, it, f, b, rows ? slot + kNB * kNB : akk, rows ? kNB : lda, slot);
-        }
+        // L_kk beside the block while others may read it
+        if (first) diag_put<TS, T>(sm.c.l, w, it, f, b, rows ? slot + kNB * kNB : akk, rows ? kNB : lda, slot);
       },
       // The rows, on the waves that have time: strips that column k - 1 is applied to
       // and column blocks solved beside sweep w, as masks (4 bits per sweep, 16 per
@@ -263,18 +263,7 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, 2) void panel_step_kernel(TS* a, 
         }
       });
   if (fail >= 0) {
-    if (first) {
-      if (rows) {
-        // the columns of the steps before the failing one, stored beside the block
-        const int w = fail / W;
-        __syncthreads();
-        for (int e = tid; e < kNB * W * w; e += NT) {
-          const int row = e / (W * w), col = e % (W * w);
-          if (col <= row && row <= fail) akk[(int64_t)row * lda + col] = slot[kNB * kNB + row * kNB + col];
-        }
-      }
-      if (tid == 0) atomicMin(info, (int32_t)(k0 + fail));
-    }
+    if (first && tid == 0) atomicMin(info, (int32_t)(k0 + fail));
     return;
   }
   if (rows && solver) {
