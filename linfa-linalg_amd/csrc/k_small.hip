@@ -49,7 +49,7 @@ __global__ __launch_bounds__(NT) void potrf_potrs_exact_batched(const SmallDesc<
                                                                 int count, int do_solve) {
   const int bi = blockIdx.x;
   if (bi >= count) return;
-  __shared__ SmallLds<T, NMAX, MCH> lds;
+  __shared__ SmallLds<T, NMAX, NT, MCH> lds;
   small_solve_one<T, NMAX, NT, MCH>(descs[bi], do_solve, lds);
 }
 
@@ -59,7 +59,7 @@ template <typename T, int NMAX, int NT, int MCH>
 __global__ __launch_bounds__(NT) void small_batch_kernel(const BatchBase<T>* __restrict__ base,
                                                          const BatchItem* __restrict__ items, int count,
                                                          int counter, int mode) {
-  __shared__ SmallLds<T, NMAX, MCH> lds;
+  __shared__ SmallLds<T, NMAX, NT, MCH> lds;
   __shared__ int s_next;
   const BatchBase<T> bb = *base;
   for (;;) {

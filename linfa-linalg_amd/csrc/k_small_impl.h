@@ -233,15 +233,16 @@ __device__ void write_back(TS* __restrict__ a, int64_t lda, int n, int fail, con
   }
 }
 
-// LDS of one small factor + solve.
-template <typename T, int NMAX, int MCH>
+// LDS of one small factor + solve on NT threads: only a single wave solves in LDS.
+template <typename T, int NMAX, int NT, int MCH>
 struct SmallLds {
   T W[(NMAX * (NMAX + 1)) / 2];
   T Ap[(NMAX * (NMAX + 1)) / 2];
   T Dg[NMAX];
-  T Bs[NMAX * MCH];
-  T Xs[NMAX * MCH];
+  T Bs[NT == 64 ? NMAX * MCH : 1];
+  T Xs[NT == 64 ? NMAX * MCH : 1];
 };
+static_assert(4 * sizeof(SmallLds<double, 64, 128, 8>) <= 160 * 1024, "four matrices of order 64 on a CU");
 
 // Both substitutions with the factor in W and Dg, for all columns of ds.b: a wave
 // takes MCH / NW columns at a time, a lane rows lane + 64 r of them in registers, so
@@ -318,7 +319,7 @@ __device__ void solve_exact(const SmallDesc<T>& ds, const T* W, const T* Dg) {
 // refinement steps of a batched mixed-precision solve need); ds.info is read:
 // a matrix whose factor failed is skipped.
 template <typename T, int NMAX, int NT, int MCH>
-__device__ void small_solve_one(const SmallDesc<T>& ds, int do_solve, SmallLds<T, NMAX, MCH>& lds) {
+__device__ void small_solve_one(const SmallDesc<T>& ds, int do_solve, SmallLds<T, NMAX, NT, MCH>& lds) {
   const int n = ds.n;
   if (n > NMAX) return;  // the host never routes a larger matrix here
   T* W = lds.W;
