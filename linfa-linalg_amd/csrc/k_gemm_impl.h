@@ -80,6 +80,9 @@ constexpr int mfma_lane_k() { return sizeof(TI) == 2 ? 8 : 1; }
 // every workgroup of a rank-k update with small k reads its C tile at the same
 // moment, after its MFMAs, and the launch waits on one HBM burst per tile.
 //
+// HOLD (beta != 0): C is read before the slabs and held in registers to the end, where the
+// sum is added to it as a whole (PRE rounds the sum's last slabs at C's size).
+//
 // TI is the operand type: T itself, or _Float16 with T = float (f16 products
 // accumulated in f32; one MFMA then takes a lane's whole 8-element fragment).
 //
@@ -91,7 +94,7 @@ template <typename TI, int ROWS>
 using NtSlab = TI[ROWS * 9 * (16 / sizeof(TI))];
 
 template <typename T, int BM, int BN, int WM, int WN, bool TRI, bool VEC, bool PRE = false, typename TI = T,
-          bool TOUT = false>
+          bool TOUT = false, bool HOLD = false>
 __device__ __forceinline__ void nt_tile_in(int M, int N, int K, T alpha, const TI* A, int64_t lda,
                                            const TI* __restrict__ B, int64_t ldb, T beta, T* C, int64_t ldc,
                                            int m0, int n0, NtSlab<TI, BM>* As, NtSlab<TI, BN>* Bs,
@@ -206,6 +209,16 @@ __device__ __forceinline__ void nt_tile_in(int M, int N, int K, T alpha, const T
   };
 
   load(0);
+  T held[HOLD ? FM : 1][HOLD ? FN : 1][4];
+  if constexpr (HOLD) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+      for (int j = 0; j < FN; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          held[i][j][r] = C[(int64_t)min(ci0 + i * 16 + MF::kRowStep * r, M - 1) * ldc + min(cj0 + j * 16, N - 1)];
+  }
   store(0);
   __syncthreads();
   for (int sl = 0; sl < nslab; ++sl) {
@@ -254,7 +267,10 @@ __device__ __forceinline__ void nt_tile_in(int M, int N, int K, T alpha, const T
         if (gi < M && gj < N && (!TRI || gi >= gj)) {
           T* c = C + (int64_t)gi * ldc + gj;
           const T v = alpha * acc[i][j][r];
-          out = (beta == T(0) || (PRE && pre)) ? v : beta * *c + v;
+          if constexpr (HOLD)
+            out = beta * held[i][j][r] + v;
+          else
+            out = (beta == T(0) || (PRE && pre)) ? v : beta * *c + v;
           *c = out;
         }
         if constexpr (TOUT) tile_out[(wm0 + i * 16 + MF::row(lane, r)) * (BN + 1) + wn0 + j * 16 + fr] = out;

@@ -74,9 +74,9 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, 2) void panel_step_kernel(TS* a, 
     const int u = blockIdx.x - nchain, ri = u / ncol, jj = u % ncol;
     if (jj > ri) return;
     const TS* p = a + (int64_t)r0 * lda + (k0 - kNB);
-    nt_tile_in<TS, 64, 64, 2, WIDE ? 4 : 2, true, VEC, sizeof(TS) == 8>(n - r0, kend - r0, kNB, TS(-1), p, lda, p, lda, TS(1),
-                                                             a + (int64_t)r0 * lda + r0, lda, 64 * ri, 64 * jj,
-                                                             sm.t.as, sm.t.bs);
+    nt_tile_in<TS, 64, 64, 2, WIDE ? 4 : 2, true, VEC, false, TS, false, true>(
+        n - r0, kend - r0, kNB, TS(-1), p, lda, p, lda, TS(1), a + (int64_t)r0 * lda + r0, lda, 64 * ri, 64 * jj,
+        sm.t.as, sm.t.bs);
     return;
   }
   __builtin_amdgcn_s_setprio(3);

@@ -471,6 +471,7 @@ __global__ __launch_bounds__(256, 2) void trsm_persistent_kernel(
     auto sweep = [&](auto divide) __attribute__((always_inline)) {
       static_for(std::make_integer_sequence<int, 4>{}, [&](auto bc) __attribute__((always_inline)) {
         constexpr int b = decltype(bc)::value;
+        T sum[4] = {T(0), T(0), T(0), T(0)};  // of these 16 columns, for the rows of later blocks
         static_for(std::make_integer_sequence<int, 16 / VL>{}, [&](auto gc) __attribute__((always_inline)) {
           constexpr int i0 = decltype(gc)::value * VL;
           vec_t l[4];
@@ -483,9 +484,11 @@ __global__ __launch_bounds__(256, 2) void trsm_persistent_kernel(
             const T u = __builtin_elementwise_fma(-l[b][v], q, rhs[b]);
             rhs[b] = fr > i ? u : rhs[b];
 #pragma unroll
-            for (int e = b + 1; e < 4; ++e) rhs[e] = __builtin_elementwise_fma(-l[e][v], q, rhs[e]);
+            for (int e = b + 1; e < 4; ++e) sum[e] = __builtin_elementwise_fma(l[e][v], q, sum[e]);
           });
         });
+#pragma unroll
+        for (int e = b + 1; e < 4; ++e) rhs[e] -= sum[e];
       });
     };
     // (pivots whose reciprocal is no normal number are divided by; those of 0 and
