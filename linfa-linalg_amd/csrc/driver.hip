@@ -39,10 +39,12 @@ hipError_t factor_steps(T* a, int64_t lda, int n, int k0, int kb, int32_t* info,
   const int end = k0 + kb;
   for (int k = k0; k < end; k += kNB) {
     const double db = std::min(kNB, n - k), below = std::max(0, n - k - kNB), pb = k > k0 ? db : 0.0;
-    const double cols = std::max(0, end - k - kNB);
+    const bool ahead = !diag_f64 && step_ahead<T>(k, k0);
+    const double cols = std::max(0, ahead ? std::min(kNB, end - k - kNB) : end - k - kNB);
     const double outs = below * cols - cols * (cols - 1.0) / 2.0;
-    LLH_PROF_ON(st, kDiagFactor, 2.0 * db * db * db / 3.0 + 2.0 * below * db * (db + pb) + 2.0 * outs * pb,
-                es * (2.0 * db * db + below * (2.0 * db + pb) + (pb > 0.0 ? 2.0 * outs : 0.0)),
+    const double rank = pb > 0.0 ? (diag_f64 ? kNB : step_rank<T>(k, k0)) : 0.0;
+    LLH_PROF_ON(st, kDiagFactor, 2.0 * db * db * db / 3.0 + 2.0 * below * db * (db + pb) + 2.0 * outs * rank,
+                es * (2.0 * db * db + below * (2.0 * db + rank) + (pb > 0.0 ? 2.0 * outs : 0.0)),
                 (diag_f64 && sizeof(T) == 4
                      ? launch_panel_step<T, double>(a, lda, n, k, k0, end, dinv, info, *stepped, beside, st)
                      : launch_panel_step<T>(a, lda, n, k, k0, end, dinv, info, *stepped, beside, st)));

@@ -38,6 +38,14 @@ inline int outer_width(int n, bool half_syrk) { return (!half_syrk && n >= kNBO_
 constexpr int kStepTail = 4096;
 inline int panel_width(int rem, int n, bool half_syrk) { return rem <= kStepTail ? rem : outer_width(n, half_syrk); }
 
+// The panel step at block column k0 applies step_rank columns before it to later block
+// columns, all of them or, with step_ahead, the next one (k_step.hip); T: the type its
+// diagonal block is factored in.
+template <typename T>
+__host__ __device__ inline bool step_ahead(int k0, int p0) { return sizeof(T) == 4 && (k0 - p0) / kNB % 2 != 0; }
+template <typename T>
+__host__ __device__ inline int step_rank(int k0, int p0) { return sizeof(T) == 8 || step_ahead<T>(k0, p0) ? kNB : 2 * kNB; }
+
 // A panel of at most so many rows is stepped through with all of them: every step's
 // launch solves the rows below as well.  With more, the steps take the panel's top
 // block alone, beside the trailing update, and the rows below follow in one launch:
