@@ -33,6 +33,12 @@ def outer_width(n):
 PEAK_HBM_GBS = 8000.0
 
 
+def panel_width(rem, n):
+    """Width of the factor's panel with rem columns left of n (csrc/llh_common.h): the
+    last 4096 are one panel."""
+    return rem if rem <= 4096 else outer_width(n)
+
+
 def solve_flops(n, m):
     return n ** 3 / 3.0 + n ** 2 / 2.0 + n / 6.0 + 2.0 * n * n * m
 
@@ -515,17 +521,17 @@ def rocprof_summary(trace_dir, fetch_dir, write_dir, n, out_md, out_json, comman
         counters[ctr] = {"copy_kib": copy, "known_kib": known_kib, "factor": factor, "launches": len(vals),
                          "avg_kib": sum(vals) / len(vals), "bytes_per_launch": sum(vals) / len(vals) * 1024 * factor}
     traffic = counters["FETCH_SIZE"]["bytes_per_launch"] + counters["WRITE_SIZE"]["bytes_per_launch"]
-    # algorithmic bytes of the trailing SYRKs of one factorization (outer panel
-    # width outer_width(n); with lookahead each SYRK leaves out the next panel's columns)
+    # algorithmic bytes of the trailing SYRKs of one factorization (panel widths
+    # panel_width(); with lookahead each SYRK leaves out the next panel's columns)
     alg = []
     k0 = 0
-    outer = outer_width(n)
     while k0 < n:
-        kb = min(outer, n - k0)
-        m3 = n - k0 - kb - min(outer, max(n - k0 - kb, 0))
+        kb = panel_width(n - k0, n)
+        m3 = n - k0 - kb - (panel_width(n - k0 - kb, n) if k0 + kb < n else 0)
         if m3 > 0:
             alg.append(8.0 * (m3 * (m3 + 1) + m3 * kb))
         k0 += kb
+    assert syrk_calls % len(alg) == 0, (syrk_calls, len(alg))
     alg_avg = sum(alg) / len(alg)
     res = {"n": n, "kernel_class": "trailing SYRK (nt_dma_kernel<double,TRI,SQ>)",
            "avg_launch_us": syrk_ns / syrk_calls / 1e3, "launches": syrk_calls,

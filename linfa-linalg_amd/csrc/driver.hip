@@ -282,10 +282,10 @@ hipError_t trsm_split(bool upper_op, bool trans, int n, const T* a, int64_t lda,
 
 }  // namespace
 
-// Blocked substitution for op(A) X = B (B row-major n x m, in place), kNB rows
-// at a time: solve the diagonal block, then subtract its contribution from the
-// rows still to come with one GEMM (the column sweep of triangular.rs:113-125,
-// done a block of rows at a time).
+// Blocked solve of op(A) X = B (B row-major n x m, in place): trsm_split, or, without
+// sync or beyond kSolveMaxCols columns, the substitution kNB rows at a time: solve the
+// diagonal block, then subtract its contribution from the rows still to come with one
+// GEMM (the column sweep of triangular.rs:113-125, done a block of rows at a time).
 template <typename T>
 hipError_t trsm_enqueue(bool upper_op, bool trans, int n, const T* a, int64_t lda, int m, T* b, int64_t ldb,
                         const T* dinv, bool dinv_t, T* dinv_work, SolveSync* sync, hipStream_t s,
@@ -369,8 +369,8 @@ bool forward_fusable(int n, int m, const Lookahead* la) {
 }
 
 // At n = 32768 with 16 right-hand sides the forward triangle after the factor
-// is ~3.5 ms (512 flag hops); fused, each panel's 16-hop triangle and product
-// run beside the trailing SYRK and only the last one trails the factor.
+// would be 1.5 ms (512 hops); fused, each panel's 16-hop triangle and product
+// run beside the trailing SYRK and only the last panel's, up to 64 hops, trail the factor.
 template <typename T>
 hipError_t factor_solve_enqueue(T* a, int64_t lda, int n, int m, T* b, int64_t ldb, T* dinv, T* y, SolveSync* sync,
                                 int32_t* info, hipStream_t s, Profiler* prof, const Lookahead* la) {

@@ -54,7 +54,8 @@ __device__ __forceinline__ T lane_value(T v, int from) {
 // Dg then hold the columns before it.
 //
 // A lane holds rows lane + 64 r and a wave the columns wave + NW i: the pending sums
-// S[j, k'] (see k_small.hip) stay in registers.  Once column k is in LDS, its successor's
+// S[j, k'] (see k_small.hip) stay in registers (on 16 waves in f64, with 128 registers
+// each, 36 are spilled; with 8 waves and none the factor takes longer, k_small.hip).  Once column k is in LDS, its successor's
 // wave brings that column up to date before any other, takes its pivot and publishes
 // it, while the rest of the sums is updated.  The sums move down by one place every NW
 // columns, so that the next column is always at place 0 (or 1).

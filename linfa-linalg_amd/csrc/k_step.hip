@@ -54,9 +54,9 @@ union StepLds {
 // An f32 factor with f64 diagonal blocks is refined afterwards and goes the f64 way.
 //
 // WIDE: eight waves, the rows on four of their own; otherwise four waves, the rows on
-// those that do not sweep.  The narrow form takes no more registers and LDS than a
-// workgroup of the trailing update (nt_dma_kernel) and so fits where one has ended:
-// the wide form, or one of 70 KB, finds no room on a CU until the whole update has
+// those that do not sweep.  The narrow form fits where a workgroup of the trailing update
+// (nt_dma_kernel) has ended, beside the other one of the CU (188 registers of 256, 66.1
+// and 65.5 KB of LDS): the wide form, or one of 70 KB, finds no room on a CU until the whole update has
 // drained (n = 16384 f64: one step's launch waited 600 to 1800 us).  Beside the update a
 // step takes 60 us (its FMAs wait for the other workgroup's f64 MFMAs), alone 19; the
 // wide form 17.  solvec n = 1500 765 us with the narrow form alone, 725 with the wide.
@@ -292,7 +292,9 @@ __global__ __launch_bounds__(WIDE ? 512 : 256, 2) void panel_step_kernel(TS* a, 
 // that every CU has one up to kRowsNarrow rows; the inverse's rows and A_k are loaded
 // before the sum.  Its registers and LDS, like a narrow step's, fit where a workgroup
 // of the trailing update has ended.  8448 x 512 f64: 119 us with 64 rows, 16 columns a
-// slab and eight waves; this form 71 us alone, 110 to 190 beside the update.  potrf
+// slab and eight waves; this form 71 us alone, 110 to 190 beside the update.  Under the
+// register bound that lets it fit, the f64 form of 64 rows spills 22 to 24 of them
+// (n = 32768: 1681 us a launch beside the update).  potrf
 // against the recursion of 64-wide panels (ms): f64 n = 16384 29.5 -> 29.0, f32 n = 12000
 // 8.65 -> 8.40, 16384 18.1 -> 17.4.
 template <typename T, bool VEC, int MT>

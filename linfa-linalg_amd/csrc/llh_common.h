@@ -67,7 +67,6 @@ constexpr int64_t kSpinLimit = 1ll << 22;
 constexpr int kMailRing = 8;
 constexpr int kMailSlot = 2 * kNB * kSolveChunkHost;
 constexpr int kMailChunks = 128;
-inline int64_t solve_chunks(int64_t m) { return (m + kSolveChunkHost - 1) / kSolveChunkHost; }
 inline int64_t solve_mail_words(int64_t chunks) { return chunks * kMailRing * kMailSlot; }
 // Tags that a launch of n rows takes: one per lap of the ring.
 inline int solve_epochs(int n) { return ((n + kNB - 1) / kNB + kMailRing - 1) / kMailRing; }
